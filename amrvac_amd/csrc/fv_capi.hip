@@ -1334,6 +1334,7 @@ static int alloc_level(amrvac_fv_ctx* c, int nblocks, int capacity, const double
     fp.dxinv[d] = 1.0 / c->dx[d];
     const double r = g.cada3_radius * c->dx[d];
     fp.rdelinv[d] = 1.0 / (r * r);
+    fp.cada3k[d] = 0.5e14 * fp.rdelinv[d];
     if (d < nd) {
       fp.invds2 = fp.invds2 + 1.0 / (c->dx[d] * c->dx[d]);
       if (c->dx[d] < fp.mindx) fp.mindx = c->dx[d];
