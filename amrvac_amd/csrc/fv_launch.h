@@ -78,12 +78,16 @@ namespace FV_NS {
 using fvc::KernelKey;
 
 
+// workgroups along z (3-D): the parts a block's planes are split into
+inline dim3 sweep_grid(const SweepArgs& a, int grid) { return dim3(grid, (a.bnz + a.zc - 1) / a.zc); }
+
 template <class P, class R, int RIEM, int LIM, int NG>
 hipError_t launch_one(const SweepArgs& a, const FVParams& fp, int grid, hipStream_t s) {
   if (a.blevel)
-    hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, true, 16>), dim3(grid), dim3(kLanes<16>), 0, s, a, fp);
+    hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, true, 16>), sweep_grid(a, grid), dim3(kLanes<16>), 0, s, a,
+                       fp);
   else
-    hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, false, 16>), dim3(grid), dim3(kLanes<16>), 0, s, a,
+    hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, false, 16>), sweep_grid(a, grid), dim3(kLanes<16>), 0, s, a,
                        fp);
   return hipGetLastError();
 }
@@ -93,7 +97,7 @@ hipError_t launch_one(const SweepArgs& a, const FVParams& fp, int grid, hipStrea
 // uniform and AMR levels
 template <class P, class R, int RIEM, int NG, int BXc>
 hipError_t launch_small(const SweepArgs& a, const FVParams& fp, int grid, hipStream_t s) {
-  hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, NG == 3 ? LIM_WENO5 : 0, NG, true, BXc>), dim3(grid),
+  hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, NG == 3 ? LIM_WENO5 : 0, NG, true, BXc>), sweep_grid(a, grid),
                      dim3(kLanes<BXc>), 0, s, a, fp);
   return hipGetLastError();
 }

@@ -8,7 +8,9 @@
 // converted to primitive variables once and staged in LDS.  In 3-D the
 // workgroup marches along z with a per-lane register window of 2*NG
 // primitive planes; x/y faces of the current plane come from LDS, the z face
-// from the window, and each z-face flux is computed once and carried.
+// from the window, and each z-face flux is computed once and carried.  On a
+// level with too few blocks to fill the GPU a block's planes are split over
+// several workgroups (blockIdx.y), each with its own window and first face.
 //
 // Per cell and stage the kernel does what finite_volume
 // (src/mod_finite_volume.t:116-339) or hancock (:19-113) plus addsource2
@@ -36,6 +38,7 @@ struct SweepArgs {
   int bx;              // block_nx(1) = block_nx(2)
   int bnz;             // block_nx(3) (1 in 2-D)
   int per_xcd;         // ceil(nblocks/8)
+  int zc;              // planes of a workgroup (3-D; bnz: the block is not split)
   int comb_mode;       // 0: init = dst, 1: init = base, 2: init = a*base + b*src,
                        // 3: init = src (base is the stage input itself)
   double comb_a, comb_b;
@@ -52,7 +55,7 @@ struct SweepArgs {
   const int* fregoff;       // [nb][2*ndim] register offset of a face, -1: none
   int nface;                // transverse cells of a face (register stride)
   int linde;                // Linde's source follows the stage (linde_kernel)
-  // CFL partials of the output (uniform level): per block the max over
+  // CFL partials of the output (uniform level): per workgroup the max over
   // cells of sum_d cmax_d/dx_d and of cmax, as getdt_courant needs them;
   // nullptr: not wanted
   double* dt_part;
@@ -294,6 +297,10 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   const size_t cells = (size_t)BX * BX * a.bnz;
   const size_t boff = (size_t)b * NW * cells;
 
+  const int nz = NDIM == 3 ? a.bnz : 1;
+  const int z0 = NDIM == 3 ? (int)blockIdx.y * a.zc : 0;  // this workgroup's planes z0 .. z1-1
+  const int z1 = NDIM == 3 ? (z0 + a.zc < nz ? z0 + a.zc : nz) : 1;
+
   // z window (3-D): Wp[m] = primitive plane k-NG+1+m (m < NG, the current
   // plane last), Wc[m] = conserved plane k+1+m as stored (FP64).  The current
   // plane's conserved state is the RK input of comb modes 2 and 3, so the
@@ -312,21 +319,21 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     for (int m = 0; m < NG; ++m) prim_of<P, R>(Wc[m], Z[NG + m], fp);
   };
   if constexpr (NDIM == 3) {
-    // prologue: planes -NG .. NG-1, halo ring of planes 0 .. NG-1, carried
-    // face -1/2
+    // prologue: planes z0-NG .. z0+NG-1, halo ring of planes z0 .. z0+NG-1,
+    // carried face z0-1/2
 #pragma unroll
-    for (int m = 0; m < NG; ++m) load_prim<P, R, NDIM, BX>(a, fp, b, tx, ty, m - NG, Wp[m]);
+    for (int m = 0; m < NG; ++m) load_prim<P, R, NDIM, BX>(a, fp, b, tx, ty, z0 + m - NG, Wp[m]);
 #pragma unroll
-    for (int m = 0; m < NG; ++m) load_cons_at<P, NDIM, BX>(a, b, tx, ty, m, Wc[m]);
+    for (int m = 0; m < NG; ++m) load_cons_at<P, NDIM, BX>(a, b, tx, ty, z0 + m, Wc[m]);
     if constexpr (HRING) {
-      for (int p = 0; p < NG && p < a.bnz; ++p)
+      for (int p = z0; p < z0 + NG && p < z1; ++p)
         for (int t = tid; t < NSTRIP; t += NTHREADS) {
           int x, y;
           strip_cell<NG, BX>(t, x, y);
           R w[NW];
           load_prim<P, R, NDIM, BX>(a, fp, b, x, y, p, w);
 #pragma unroll
-          for (int iw = 0; iw < NW; ++iw) hring[p][iw][t] = w[iw];
+          for (int iw = 0; iw < NW; ++iw) hring[p % NG][iw][t] = w[iw];
         }
     }
     if constexpr (!HANCOCK) {
@@ -337,8 +344,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     if constexpr (HRING) __syncthreads();
   }
 
-  const int nz = NDIM == 3 ? a.bnz : 1;
-  for (int k = 0; k < nz; ++k) {
+  for (int k = z0; k < z1; ++k) {
     const size_t o = boff + ((size_t)k * BX + ty) * BX + tx;
     double cons_k[NW];  // wCT of this lane's cell
     double acc[NW];
@@ -414,7 +420,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     __syncthreads();
     if constexpr (HRING) {
       // halo of plane k+NG into the ring slot just copied out
-      if (k + NG < nz) {
+      if (k + NG < z1) {
         const int slot = k % NG;
         // by the upper waves: the lower ones take the partial face pass
         const int th = NTHREADS == 256 ? (tid + 128) % NTHREADS : tid;
@@ -615,8 +621,9 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       if (tid == 0) {
         double m = dtr[0][0], c = dtr[1][0];
         for (int i = 1; i < NTHREADS / 64; ++i) { m = fmax(m, dtr[0][i]); c = fmax(c, dtr[1][i]); }
-        a.dt_part[2 * b] = m;
-        a.dt_part[2 * b + 1] = c;
+        const int w = b * (int)gridDim.y + (int)blockIdx.y;
+        a.dt_part[2 * w] = m;
+        a.dt_part[2 * w + 1] = c;
       }
     }
   }
