@@ -342,7 +342,10 @@ __global__ void __launch_bounds__(NTHREADS) restrict_kernel(double* w, int nw, i
   const size_t cells = (size_t)BXr * BXr * bnz;
   const double cofi = 1.0 / double(1 << NDIM);
   const int total = cnt[0] * cnt[1] * cnt[2];
-  for (int c = threadIdx.x; c < total; c += NTHREADS) {
+  // a lane takes one cell and two variables, all of whose fine cells are
+  // loaded before the first is summed
+  for (int q = threadIdx.x; q < total * ((nw + 1) / 2); q += NTHREADS) {
+    const int c = q % total, iw0 = 2 * (q / total);
     const int g[3] = {lo[0] + c % cnt[0], lo[1] + (c / cnt[0]) % cnt[1], lo[2] + c / (cnt[0] * cnt[1])};
     int gn[3] = {0, 0, 0}, f[3] = {0, 0, 0}, cidx = 0;
     for (int d = 0; d < NDIM; ++d) {
@@ -352,81 +355,116 @@ __global__ void __launch_bounds__(NTHREADS) restrict_kernel(double* w, int nw, i
       f[d] = 2 * (gn[d] - (ic - 1) * (n[d] / 2));
     }
     const int F = nchild[((size_t)C * nnb + k) * (1 << NDIM) + cidx];
-    const double* wf = w + (size_t)F * nw * cells;
+    const double* wf = w + (size_t)F * nw * cells + ((size_t)f[2] * BXr + f[1]) * BXr + f[0];
     double* wv = w + (size_t)V * nw * cells + ((size_t)gn[2] * BXr + gn[1]) * BXr + gn[0];
-    for (int iw = 0; iw < nw; ++iw) {
-      double sum = 0.0;
-      bool first = true;
-      for (int dk = 0; dk <= (NDIM > 2 ? 1 : 0); ++dk)
-        for (int dj = 0; dj <= 1; ++dj)
-          for (int di = 0; di <= 1; ++di) {
-            const double v = wf[iw * cells + ((size_t)(f[2] + dk) * BXr + (f[1] + dj)) * BXr + f[0] + di];
-            sum = first ? v : sum + v;
-            first = false;
-          }
-      wv[iw * cells] = sum * cofi;
+    const bool two = iw0 + 1 < nw;
+    double v[2][1 << NDIM];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < (1 << NDIM); ++e)
+        v[j][e] = wf[(size_t)(two ? iw0 + j : iw0) * cells + ((e >> 2) * BXr + ((e >> 1) & 1)) * BXr + (e & 1)];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      double sum = v[j][0];
+#pragma unroll
+      for (int e = 1; e < (1 << NDIM); ++e) sum = sum + v[j][e];
+      if (j == 0 || two) wv[(iw0 + j) * cells] = sum * cofi;
     }
   }
 }
 
 // one cell of the coarse representation of fine block F (1-based index p of
-// the (n/2 + 2ng)^ndim coarse grid around F), variable iw, as bc_prolong
-// sees it: physical boundary rule on the coarse grid where F touches the
-// boundary (bc_phys), the mean of F's own fine cells inside F, and the
-// coarse neighbour's data (its interior or, through its neighbour table,
-// its same-level or restricted ghost cells) elsewhere
+// the (n/2 + 2ng)^ndim coarse grid around F), as bc_prolong sees it: physical
+// boundary rule on the coarse grid where F touches the boundary (bc_phys), the
+// mean of F's own fine cells inside F, and the coarse neighbour's data (its
+// interior or, through its neighbour table, its same-level or restricted
+// ghost cells) elsewhere.  Resolved once for all variables: get(iw) reads one.
 template <int NDIM>
-__device__ double psc_value(const SweepArgs& a, int nw, int ng, int F, int C, const int* icF, const int* iC,
-                            const bool (*bnd)[2], int p0, int p1, int p2, int iw) {
-  const int BXr = a.bx;  // block_nx(1) = block_nx(2)
-  const int n[3] = {BXr, BXr, a.bnz};
-  int q[3] = {p0, p1, p2};
-  double sign = 1.0;
-  bool inside = true;
-  for (int d = 0; d < NDIM; ++d) {
-    const int clo = ng + 1, chi = ng + n[d] / 2;
-    if (q[d] < clo && bnd[d][0]) {
-      const int tp = a.bc[2 * d];
-      if (tp == 2) q[d] = clo;
-      else { q[d] = 2 * clo - 1 - q[d]; if (tp == 4) sign = -sign; }
-    } else if (q[d] > chi && bnd[d][1]) {
-      const int tp = a.bc[2 * d + 1];
-      if (tp == 2) q[d] = chi;
-      else { q[d] = 2 * chi + 1 - q[d]; if (tp == 4) sign = -sign; }
+struct PscCell {
+  const double* p;  // variable 0 of the cell, or of the first of 2^ndim fine cells
+  size_t cells;
+  int bx, plane;
+  bool mean;
+  double sign;
+  __device__ __forceinline__ PscCell(const SweepArgs& a, int nw, int ng, int F, int C, const int* icF, const int* iC,
+                                     const bool (*bnd)[2], const int* p0) {
+    const int BXr = a.bx;  // block_nx(1) = block_nx(2)
+    const int n[3] = {BXr, BXr, a.bnz};
+    int q[3] = {p0[0], p0[1], p0[2]};
+    sign = 1.0;
+    mean = true;
+    for (int d = 0; d < NDIM; ++d) {
+      const int clo = ng + 1, chi = ng + n[d] / 2;
+      if (q[d] < clo && bnd[d][0]) {
+        const int tp = a.bc[2 * d];
+        if (tp == 2) q[d] = clo;
+        else { q[d] = 2 * clo - 1 - q[d]; if (tp == 4) sign = -sign; }
+      } else if (q[d] > chi && bnd[d][1]) {
+        const int tp = a.bc[2 * d + 1];
+        if (tp == 2) q[d] = chi;
+        else { q[d] = 2 * chi + 1 - q[d]; if (tp == 4) sign = -sign; }
+      }
+      if (q[d] < clo || q[d] > chi) mean = false;
     }
-    if (q[d] < clo || q[d] > chi) inside = false;
+    bx = BXr;
+    plane = BXr * BXr;
+    cells = (size_t)plane * a.bnz;
+    int x[3] = {0, 0, 0};
+    int sb = F;
+    if (mean) {
+      for (int d = 0; d < NDIM; ++d) x[d] = 2 * (q[d] - (ng + 1));
+    } else {
+      for (int d = 0; d < NDIM; ++d) x[d] = q[d] + (icF[d] - 1) * (n[d] / 2) + n[d] * iC[d] - ng - 1;
+      double s2;
+      sb = locate<NDIM>(a, C, x[0], x[1], x[2], s2);
+      sign = sign * s2;
+    }
+    p = a.src + (size_t)sb * nw * cells + (size_t)x[2] * plane + x[1] * bx + x[0];
   }
-  const size_t cells = (size_t)BXr * BXr * a.bnz;
-  if (inside) {
-    int f[3] = {0, 0, 0};
-    for (int d = 0; d < NDIM; ++d) f[d] = 2 * (q[d] - (ng + 1));
-    const double* wf = a.src + (size_t)F * nw * cells + iw * cells;
+  __device__ __forceinline__ double get(int iw) const {
+    const double* w = p + iw * cells;
+    if (!mean) return sign * w[0];
     double sum = 0.0;
     bool first = true;
+#pragma unroll
     for (int dk = 0; dk <= (NDIM > 2 ? 1 : 0); ++dk)
+#pragma unroll
       for (int dj = 0; dj <= 1; ++dj)
+#pragma unroll
         for (int di = 0; di <= 1; ++di) {
-          const double v = wf[((size_t)(f[2] + dk) * BXr + (f[1] + dj)) * BXr + f[0] + di];
+          const double v = w[dk * plane + dj * bx + di];
           sum = first ? v : sum + v;
           first = false;
         }
     return sign * (sum * (1.0 / double(1 << NDIM)));
   }
-  int x[3] = {0, 0, 0};
-  for (int d = 0; d < NDIM; ++d) x[d] = q[d] + (icF[d] - 1) * (n[d] / 2) + n[d] * iC[d] - ng - 1;
-  double s2;
-  const int sb = locate<NDIM>(a, C, x[0], x[1], x[2], s2);
-  return sign * s2 * a.src[(size_t)sb * nw * cells + iw * cells + ((size_t)x[2] * BXr + x[1]) * BXr + x[0]];
-}
+};
 
 // Ghost cells of a fine block facing a coarser neighbour: interpolation_linear
 // (src/mod_ghostcells_update.t:1381-1525, slab_uniform, conserved variables)
 // from the coarse representation with limited slopes, as bc_prolong
 // (:1261-1339) and bc_fill_prolong (:1103-1154) assemble it.
+// One workgroup per ghost region (face, edge or corner of a block).  The
+// coarse cells under the region and their axis neighbours are resolved and
+// read once each into LDS; the lanes then take (fine cell, variable) pairs.
+// Bound by the latency of the lookups: with one lane per fine cell, resolving
+// every stencil cell of every variable anew (2 ndim + 1 lookups each), it took
+// 384 us for 3186 blocks of 8^3, now 92.
+constexpr int kPrZ = 16;  // planes of a region staged at a time
+// LDS cells of a staged region: ghost direction at most (ng + 1)/2 + 1 coarse
+// cells, tangential ones n/2 + 1, and one more on each side
+inline size_t prolong_tile_cells(int ndim, int bx, int bnz, int ng) {
+  const int gh = (ng + 1) / 2 + 3, tx = bx / 2 + 3, tz = (bnz < kPrZ ? bnz : kPrZ) / 2 + 3;
+  const int mx = std::max(gh, tx), mz = std::max(gh, tz);
+  if (ndim == 2) return (size_t)gh * mx;
+  return (size_t)gh * mx * std::max(mx, mz);
+}
 template <int NDIM>
 __global__ void __launch_bounds__(NTHREADS) prolong_kernel(SweepArgs a, double* w, int nw, int ng, int nnb,
                                                            const int4* task, const int2* task2, const int* ntype,
                                                            const int* level, const double* xlo, FVParams fp) {
+  extern __shared__ double tile[];  // [nw][coarse cells]
   const int BXr = a.bx;  // block_nx(1) = block_nx(2)
   const int4 t = task[blockIdx.x];
   const int2 t2 = task2[blockIdx.x];
@@ -461,30 +499,67 @@ __global__ void __launch_bounds__(NTHREADS) prolong_kernel(SweepArgs a, double* 
     xFimin[d] = rpxmin - double(ng) * dxFi[d];
     xComin[d] = rpxmin - double(ng) * dxCo[d];
   }
+  // coarse cell (1-based) under fine ghost cell g of dimension d
+  auto coarse = [&](int d, int g, double& xFi) {
+    xFi = xFimin[d] + (double(g + ng + 1) - 0.5) * dxFi[d];
+    return int((xFi - xComin[d]) * invdxCo[d]) + 1;
+  };
   const size_t cells = (size_t)BXr * BXr * a.bnz;
-  const int total = cnt[0] * cnt[1] * cnt[2];
-  for (int c = threadIdx.x; c < total; c += NTHREADS) {
-    const int g[3] = {lo[0] + c % cnt[0], lo[1] + (c / cnt[0]) % cnt[1], lo[2] + c / (cnt[0] * cnt[1])};
-    int co[3] = {1, 1, 1};
-    double eta[3] = {0, 0, 0};
-    for (int d = 0; d < NDIM; ++d) {
-      const double xFi = xFimin[d] + (double(g[d] + ng + 1) - 0.5) * dxFi[d];
-      co[d] = int((xFi - xComin[d]) * invdxCo[d]) + 1;
-      const double xCo = xComin[d] + (double(co[d]) - 0.5) * dxCo[d];
-      eta[d] = (xFi - xCo) * invdxCo[d];
+  const int zlo = lo[2], zcnt = cnt[2];
+  for (int zc = 0; zc < zcnt; zc += kPrZ) {
+    if (NDIM == 3) {
+      lo[2] = zlo + zc;
+      cnt[2] = zcnt - zc < kPrZ ? zcnt - zc : kPrZ;
     }
-    int gn[3] = {0, 0, 0};
-    for (int d = 0; d < NDIM; ++d) gn[d] = g[d] - i[d] * n[d];
-    double* wv = w + (size_t)V * nw * cells + ((size_t)gn[2] * BXr + gn[1]) * BXr + gn[0];
-    for (int iw = 0; iw < nw; ++iw) {
-      const double c0 = psc_value<NDIM>(a, nw, ng, F, C, icF, iC, bnd, co[0], co[1], co[2], iw);
+    int tb[3] = {1, 1, 1}, ts[3] = {1, 1, 1};  // first coarse cell and extent of the tile
+    for (int d = 0; d < NDIM; ++d) {
+      double xf;
+      tb[d] = coarse(d, lo[d], xf) - 1;
+      ts[d] = coarse(d, lo[d] + cnt[d] - 1, xf) + 1 - tb[d] + 1;
+    }
+    const int nt = ts[0] * ts[1] * ts[2];
+    if (zc) __syncthreads();
+    // four variables per lane: the lookup is shared by them
+    for (int q = threadIdx.x; q < nt * ((nw + 3) / 4); q += blockDim.x) {
+      const int c = q % nt, iw0 = 4 * (q / nt);
+      const int e[3] = {c % ts[0], (c / ts[0]) % ts[1], c / (ts[0] * ts[1])};
+      int out = 0, p[3] = {1, 1, 1};
+      for (int d = 0; d < NDIM; ++d) {
+        out += e[d] == 0 || e[d] == ts[d] - 1;
+        p[d] = tb[d] + e[d];
+      }
+      if (out > 1) continue;  // the slopes reach along the axes only
+      const PscCell<NDIM> pc(a, nw, ng, F, C, icF, iC, bnd, p);
+      double v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = pc.get(iw0 + j < nw ? iw0 + j : iw0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (iw0 + j < nw) tile[(iw0 + j) * nt + c] = v[j];
+    }
+    __syncthreads();
+    const int total = cnt[0] * cnt[1] * cnt[2];
+    for (int q = threadIdx.x; q < total * nw; q += blockDim.x) {
+      const int iw = q / total, c = q % total;
+      const int g[3] = {lo[0] + c % cnt[0], lo[1] + (c / cnt[0]) % cnt[1], lo[2] + c / (cnt[0] * cnt[1])};
+      int l = 0, st = 1, sd[3] = {0, 0, 0}, gn[3] = {0, 0, 0};
+      double eta[3] = {0, 0, 0};
+      for (int d = 0; d < NDIM; ++d) {
+        double xFi;
+        const int co = coarse(d, g[d], xFi);
+        const double xCo = xComin[d] + (double(co) - 0.5) * dxCo[d];
+        eta[d] = (xFi - xCo) * invdxCo[d];
+        l += (co - tb[d]) * st;
+        sd[d] = st;
+        st *= ts[d];
+        gn[d] = g[d] - i[d] * n[d];
+      }
+      const double* tw = tile + iw * nt + l;
+      const double c0 = tw[0];
       double val = c0;
       for (int d = 0; d < NDIM; ++d) {
-        int h[3] = {co[0], co[1], co[2]}, p[3] = {co[0], co[1], co[2]};
-        h[d] -= 1;
-        p[d] += 1;
-        const double slopeL = c0 - psc_value<NDIM>(a, nw, ng, F, C, icF, iC, bnd, h[0], h[1], h[2], iw);
-        const double slopeR = psc_value<NDIM>(a, nw, ng, F, C, icF, iC, bnd, p[0], p[1], p[2], iw) - c0;
+        const double slopeL = c0 - tw[-sd[d]];
+        const double slopeR = tw[sd[d]] - c0;
         const double slopeC = 0.5 * (slopeR + slopeL);
         const double signC = copysign(1.0, slopeC);
         const double m1 = fabs(slopeC) < signC * slopeL ? fabs(slopeC) : signC * slopeL;
@@ -492,7 +567,7 @@ __global__ void __launch_bounds__(NTHREADS) prolong_kernel(SweepArgs a, double* 
         const double slope = signC * (0.0 > m2 ? 0.0 : m2);
         val = val + slope * eta[d];
       }
-      wv[iw * cells] = val;
+      w[(size_t)V * nw * cells + iw * cells + ((size_t)gn[2] * BXr + gn[1]) * BXr + gn[0]] = val;
     }
   }
 }
@@ -605,8 +680,11 @@ __device__ __forceinline__ double cell_value(const SweepArgs& a, int nw, int b, 
 // neighbour is coarser or finer (the level-jump rule, :5616-5641).  One
 // workgroup per block; div B of the block and its one-cell rim in LDS.
 // Built without contraction, so every build rounds like the oracle.
+// Bound by address arithmetic and the latency of the lookups (six field values
+// per rim cell): the cross-section is a compile-time constant and the block's
+// neighbours are read into LDS once (3186 blocks of 8^3: 142 to 120 us).
 constexpr int kLindeLds = 7800;  // doubles: (bx+2)^2 (bnz+2) for bx <= 16, bnz <= 22
-template <class P>
+template <class P, int bx>
 __global__ void __launch_bounds__(NTHREADS) linde_kernel(SweepArgs a, FVParams fp, const int* __restrict__ ntype,
                                                          int nnb, double* __restrict__ dst) {
   constexpr int NDIM = P::NDIM, NW = P::NW;
@@ -620,17 +698,31 @@ __global__ void __launch_bounds__(NTHREADS) linde_kernel(SweepArgs a, FVParams f
     }
     fp.invds2 = fp.invds2 * sc2;
   }
-  const int bx = a.bx, bz = NDIM == 3 ? a.bnz : 1;
-  const int ex = bx + 2, ez = NDIM == 3 ? bz + 2 : 1;
+  constexpr int NNB = NDIM == 3 ? 27 : 9;
+  const int bz = NDIM == 3 ? a.bnz : 1;
+  constexpr int ex = bx + 2;
+  const int ez = NDIM == 3 ? bz + 2 : 1;
   __shared__ double divb[kLindeLds];
+  __shared__ int nbrs[NNB];
+  if (threadIdx.x < NNB) nbrs[threadIdx.x] = a.nbr[(size_t)b * NNB + threadIdx.x];
+  __syncthreads();
+  const size_t cells = (size_t)bx * bx * a.bnz;
+  // field component v of a cell within two of the block (cell_value)
+  auto field = [&](int x, int y, int z, int v) {
+    const int dx = x < 0 ? -1 : (x >= bx ? 1 : 0), dy = y < 0 ? -1 : (y >= bx ? 1 : 0);
+    const int dz = NDIM == 3 ? (z < 0 ? -1 : (z >= bz ? 1 : 0)) : 0;
+    const int nb = nbrs[(NDIM == 3 ? 9 * (dz + 1) : 0) + 3 * (dy + 1) + dx + 1];
+    if (nb < 0) return cell_value<NDIM>(a, NW, b, x, y, z, v);
+    return a.src[((size_t)nb * NW + v) * cells + ((z - dz * bz) * bx + (y - dy * bx)) * bx + (x - dx * bx)];
+  };
   for (int c = threadIdx.x; c < ex * ex * ez; c += NTHREADS) {
     const int x = c % ex - 1, y = (c / ex) % ex - 1, z = NDIM == 3 ? c / (ex * ex) - 1 : 0;
     double d = 0.0;
 #pragma unroll
     for (int dd = 0; dd < NDIM; ++dd) {
       const int hx = dd == 0, hy = dd == 1, hz = dd == 2;
-      const double bp = cell_value<NDIM>(a, NW, b, x + hx, y + hy, z + hz, P::MAG + dd);
-      const double bm = cell_value<NDIM>(a, NW, b, x - hx, y - hy, z - hz, P::MAG + dd);
+      const double bp = field(x + hx, y + hy, z + hz, P::MAG + dd);
+      const double bm = field(x - hx, y - hy, z - hz, P::MAG + dd);
       d = d + 0.5 * (bp - bm) * fp.dxinv[dd];
     }
     divb[c] = d;
@@ -649,7 +741,6 @@ __global__ void __launch_bounds__(NTHREADS) linde_kernel(SweepArgs a, FVParams f
         }
       }
   }
-  const size_t cells = (size_t)bx * bx * a.bnz;
   double* wb = dst + (size_t)b * NW * cells;
   const double* wct = a.src + (size_t)b * NW * cells;
   int crash = 0;
@@ -683,7 +774,18 @@ hipError_t launch_linde(const SweepArgs& a, const FVParams& fp, const int* ntype
   if constexpr (!P::MHD || P::NDIM < 2) {
     return hipErrorInvalidValue;
   } else {
-    hipLaunchKernelGGL((linde_kernel<P>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+    if (a.bx == 16) {
+      hipLaunchKernelGGL((linde_kernel<P, 16>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+    } else if constexpr (P::NDIM == 3) {
+      if (a.bx == 8)
+        hipLaunchKernelGGL((linde_kernel<P, 8>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+      else if (a.bx == 10)
+        hipLaunchKernelGGL((linde_kernel<P, 10>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+      else
+        return hipErrorInvalidValue;
+    } else {
+      return hipErrorInvalidValue;
+    }
     return hipGetLastError();
   }
 }
@@ -1410,11 +1512,15 @@ static int getbc_amr(amrvac_fv_ctx* c, int slot) {
   if (c->npt) {
     fvc::SweepArgs a = base_args(c);
     a.src = c->slot[slot];
+    // one wave per region, four where a face of a 3-D block of 16^2 columns has
+    // 16 times as many values as lanes
+    const int lanes = nd == 3 && c->bx == 16 ? 256 : 64;
+    const size_t lds = fv::prolong_tile_cells(nd, c->bx, c->bnz, ng) * c->nw * sizeof(double);
     if (nd == 2)
-      hipLaunchKernelGGL((fv::prolong_kernel<2>), dim3(c->npt), dim3(fvc::NTHREADS), 0, c->stream, a, c->slot[slot],
+      hipLaunchKernelGGL((fv::prolong_kernel<2>), dim3(c->npt), dim3(lanes), lds, c->stream, a, c->slot[slot],
                          c->nw, ng, c->nnb, c->d_ptask, c->d_ptask2, c->d_ntype, c->d_level, c->d_xlo, c->fp);
     else
-      hipLaunchKernelGGL((fv::prolong_kernel<3>), dim3(c->npt), dim3(fvc::NTHREADS), 0, c->stream, a, c->slot[slot],
+      hipLaunchKernelGGL((fv::prolong_kernel<3>), dim3(c->npt), dim3(lanes), lds, c->stream, a, c->slot[slot],
                          c->nw, ng, c->nnb, c->d_ptask, c->d_ptask2, c->d_ntype, c->d_level, c->d_xlo, c->fp);
     HIPCHK(hipGetLastError());
   }
