@@ -728,6 +728,25 @@ __device__ __forceinline__ void hlld_flux(const R* wLC, const R* wRC, const R* w
   }
 }
 
+// Both primitive face states with a TVD limiter; C0: index of cell i in st
+template <class P, class R, int ID, int LIM, int C0>
+__device__ __forceinline__ void tvd_states(const R (*st)[P::NW], const FVParams& fp, R* wL, R* wR) {
+#pragma unroll
+  for (int iw = 0; iw < P::NW; ++iw) {
+    if constexpr (LIM == LIM_CADA3 && kFast64<R>) {
+      cada3_face64(fp, ID, st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], wL[iw], wR[iw]);
+    } else {
+      const R dm = st[C0][iw] - st[C0 - 1][iw];
+      const R d0 = st[C0 + 1][iw] - st[C0][iw];
+      const R dp = st[C0 + 2][iw] - st[C0 + 1][iw];
+      R ldw, rdw;
+      face_limit<R, LIM>(LIM, dm, d0, dp, R(fp.rdelinv[ID]), ldw, rdw);
+      wL[iw] = st[C0][iw] + R(0.5) * ldw;
+      wR[iw] = st[C0 + 1][iw] - R(0.5) * rdw;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // one face: reconstruct_LR (src/mod_finite_volume.t:1110-1228), modify_wLR
 // (GLM, src/mhd/mod_mhd_phys.t:6326-6377), fluxes, bounds and the Riemann
@@ -770,22 +789,32 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
 #pragma unroll
       for (int iw = 0; iw < NW; ++iw) { wLp[iw] = tl[iw]; wRp[iw] = tr[iw]; }
     }
-  } else if constexpr (LIM == LIM_CADA3 && kFast64<R>) {
-#pragma unroll
-    for (int iw = 0; iw < NW; ++iw)
-      cada3_face64(fp, ID, st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], wLp[iw], wRp[iw]);
-  } else {
-    const R rdel = R(fp.rdelinv[ID]);
+  } else if constexpr (LIM == 0 && std::is_same<R, float>::value) {
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) {
       const R dm = st[C0][iw] - st[C0 - 1][iw];
       const R d0 = st[C0 + 1][iw] - st[C0][iw];
       const R dp = st[C0 + 2][iw] - st[C0 + 1][iw];
       R ldw, rdw;
-      face_limit<R, LIM>(fp.limiter, dm, d0, dp, rdel, ldw, rdw);
+      face_limit<R, 0>(fp.limiter, dm, d0, dp, R(fp.rdelinv[ID]), ldw, rdw);
       wLp[iw] = st[C0][iw] + R(0.5) * ldw;
       wRp[iw] = st[C0 + 1][iw] - R(0.5) * rdw;
     }
+  } else if constexpr (LIM == 0) {
+    // the limiter chosen once per face, not per variable
+    switch (fp.limiter) {
+      case LIM_MINMOD: tvd_states<P, R, ID, LIM_MINMOD, C0>(st, fp, wLp, wRp); break;
+      case LIM_WOODWARD: tvd_states<P, R, ID, LIM_WOODWARD, C0>(st, fp, wLp, wRp); break;
+      case LIM_MCBETA: tvd_states<P, R, ID, LIM_MCBETA, C0>(st, fp, wLp, wRp); break;
+      case LIM_SUPERBEE: tvd_states<P, R, ID, LIM_SUPERBEE, C0>(st, fp, wLp, wRp); break;
+      case LIM_VANLEER: tvd_states<P, R, ID, LIM_VANLEER, C0>(st, fp, wLp, wRp); break;
+      case LIM_ALBADA: tvd_states<P, R, ID, LIM_ALBADA, C0>(st, fp, wLp, wRp); break;
+      case LIM_KOREN: tvd_states<P, R, ID, LIM_KOREN, C0>(st, fp, wLp, wRp); break;
+      case LIM_CADA: tvd_states<P, R, ID, LIM_CADA, C0>(st, fp, wLp, wRp); break;
+      default: tvd_states<P, R, ID, LIM_CADA3, C0>(st, fp, wLp, wRp); break;
+    }
+  } else {
+    tvd_states<P, R, ID, LIM, C0>(st, fp, wLp, wRp);
   }
   R wLC[NW], wRC[NW];
   const R inv_g1 = R(fp.inv_gamma_1);
