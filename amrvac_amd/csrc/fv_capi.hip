@@ -1361,6 +1361,17 @@ int amrvac_fv_set_mesh(amrvac_fv_ctx* c, int nblocks, const double* dx, const in
   return alloc_level(c, nblocks, nblocks, dx, neighbor, bc);
 }
 
+// the largest FP32 number whose FP32 product with r > 0 is at most 1
+static float unit_threshold(float r) {
+  float s = 1.0f / r;
+  while (s * r > 1.0f) s = std::nextafterf(s, 0.0f);
+  while (true) {
+    const float n = std::nextafterf(s, HUGE_VALF);
+    if (!(n * r <= 1.0f) || n == s) return s;
+    s = n;
+  }
+}
+
 // state slots with room for `capacity` blocks (leaves + virtual ghost
 // blocks), work buffers, the sweep's neighbour table and the scheme
 // constants of the level-1 cell size dx
@@ -1438,6 +1449,7 @@ static int alloc_level(amrvac_fv_ctx* c, int nblocks, int capacity, const double
     const double r = g.cada3_radius * c->dx[d];
     fp.rdelinv[d] = 1.0 / (r * r);
     fp.cada3k[d] = 0.5e14 * fp.rdelinv[d];
+    fp.cada3t[d] = unit_threshold((float)fp.rdelinv[d]);
     if (d < nd) {
       fp.invds2 = fp.invds2 + 1.0 / (c->dx[d] * c->dx[d]);
       if (c->dx[d] < fp.mindx) fp.mindx = c->dx[d];

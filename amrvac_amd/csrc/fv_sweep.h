@@ -227,6 +227,7 @@ __device__ __forceinline__ void level_params(const SweepArgs& a, int b, FVParams
     fp.dxinv[d] = fp.dxinv[d] * sc;
     fp.rdelinv[d] = fp.rdelinv[d] * sc2;
     fp.cada3k[d] = fp.cada3k[d] * sc2;
+    fp.cada3t[d] = fp.cada3t[d] / sc2;
     dq[d] = dq[d] * sc;
   }
   fp.invds2 = fp.invds2 * sc2;
