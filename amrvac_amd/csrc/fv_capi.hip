@@ -91,7 +91,6 @@ struct amrvac_fv_ctx {
   // CFL partials of ps left by the last stage that wrote it (uniform level,
   // production precision): getdt of ps then only reduces them
   double* d_dtp = nullptr;
-  int n_dtp = 0;  // partials (workgroups of that stage)
   bool dt_valid = false;
   bool slot0_exposed = false;  // ps handed out by amrvac_fv_slot_pointer
   double* d_red2 = nullptr;   // final reduction
@@ -1416,7 +1415,7 @@ static int alloc_level(amrvac_fv_ctx* c, int nblocks, int capacity, const double
       (!c->d_crash && hipMalloc(&c->d_crash, sizeof(int)) != hipSuccess) ||
       !ensure_buf(&c->d_red, &c->red_cap, (size_t)nblocks * 2 * (c->nw > 1 ? c->nw : 1)) ||
       (!c->d_red2 && hipMalloc(&c->d_red2, sizeof(double) * 3) != hipSuccess) || !ensure_pin(c, kPinFlags + nblocks) ||
-      !ensure_buf(&c->d_dtp, &c->dtp_cap, (size_t)nblocks * 2 * 4) ||
+      !ensure_buf(&c->d_dtp, &c->dtp_cap, (size_t)nblocks * 2) ||
       !ensure_buf(&c->d_stage, &c->stage_cap, (size_t)nblocks * c->nw * c->cells_g)) {
     free_level(c);
     return fail(AMRVAC_FV_ENOMEM, "work buffer allocation failed");
@@ -1553,10 +1552,10 @@ static int fix_conserve_amr(amrvac_fv_ctx* c, int slot) {
   return AMRVAC_FV_OK;
 }
 
-// reduction of the CFL maxima part[2*npart]: their max and the
+// reduction of the CFL maxima part[2*nb]: their max and the
 // small-value flag into fin[3], copied to the host; dt and cmax from them
 static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, double* cmax_out, double* part,
-                        int npart, double* fin);
+                        double* fin);
 
 // dt of state u: per-block maxima into part[2*nb], then getdt_reduce
 static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, double* dtmin_out, double* cmax_out,
@@ -1564,12 +1563,12 @@ static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, doub
   hipError_t e = with_phys<GetdtOp>(c, u, c->nb, c->bx, c->bnz, (const fvc::FVParams*)&c->fp, (const int*)c->d_level,
                                     part, c->d_crash, c->stream);
   if (e != hipSuccess) return fail(AMRVAC_FV_EHIP, std::string("getdt launch: ") + hipGetErrorString(e));
-  return getdt_reduce(c, courantpar, dtmin_out, cmax_out, part, c->nb, fin);
+  return getdt_reduce(c, courantpar, dtmin_out, cmax_out, part, fin);
 }
 
 static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, double* cmax_out, double* part,
-                        int npart, double* fin) {
-  hipLaunchKernelGGL(fv::reduce_max2_kernel, dim3(1), dim3(fvc::NTHREADS), 0, c->stream, part, npart, fin,
+                        double* fin) {
+  hipLaunchKernelGGL(fv::reduce_max2_kernel, dim3(1), dim3(fvc::NTHREADS), 0, c->stream, part, c->nb, fin,
                      (const int*)c->d_crash);
   HIPCHK(hipGetLastError());
   const double* r = reinterpret_cast<const double*>(c->h_pin);
@@ -1594,10 +1593,13 @@ static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, 
 // take about 1.6 times as long as one.  The split with the smallest of
 //   rounds of workgroups x time of one
 // is taken, in parts of at least 4 planes (105 blocks of 16^3, MHD: 133 us for
-// a stage in one part, 55 us in four).
+// a stage in one part, 55 us in four).  The mixed form's blocks stay whole: its
+// carried first z face is rounded apart from the others (the compiler's choice
+// of fused products), so a split would change its results.
 static int stage_zc(const amrvac_fv_ctx* c) {
   if (c->cfg.ndim != 3) return 1;
-  const int ncu = 256, per_cu = c->bx == 16 ? (c->cfg.precision == AMRVAC_FV_PREC_MIXED ? 3 : 2) : 4;
+  if (c->cfg.precision == AMRVAC_FV_PREC_MIXED) return c->bnz;
+  const int ncu = 256, per_cu = c->bx == 16 ? 2 : 4;
   int best = c->bnz;
   double tbest = 1e30;
   for (int nch = 1; nch <= 4; nch *= 2) {
@@ -1646,6 +1648,7 @@ static int stage_core(amrvac_fv_ctx* c, int method, double dtfactor, double dt, 
   const double qdt = dtfactor * dt;
   a.qdt = qdt;
   a.zc = stage_zc(c);
+  a.src_al16 = reinterpret_cast<uintptr_t>(src) % 16 == 0;
   for (int d = 0; d < 3; ++d) a.dq[d] = -qdt / c->dx[d];
   a.ch = cmax_global;
   // add_source_glm psi decay factor, src/mhd/mod_mhd_phys.t:5491-5495
@@ -1675,10 +1678,7 @@ static int stage_core(amrvac_fv_ctx* c, int method, double dtfactor, double dt, 
   a.linde = linde ? 1 : 0;
   const bool fuse_dt = dst_slot == 0 && !c->amr && c->bx == 16 && c->nws == 0 && !linde &&
                        c->cfg.precision == AMRVAC_FV_PREC_MIXED && !c->slot0_exposed;
-  if (fuse_dt) {
-    a.dt_part = c->d_dtp;
-    c->n_dtp = c->nb * ((c->bnz + a.zc - 1) / a.zc);
-  }
+  if (fuse_dt) a.dt_part = c->d_dtp;
   if (dst_slot == 0 || dst_slot < 0) c->dt_valid = false;
   if (crash_out) HIPCHK(hipMemsetAsync(c->d_crash, 0, sizeof(int), c->stream));
   const int grid = 8 * a.per_xcd;
@@ -1851,7 +1851,7 @@ int amrvac_fv_getdt(amrvac_fv_ctx* c, int slot, double courantpar, double* dtmin
   if (!c || !check_slot(slot)) return fail(AMRVAC_FV_EINVAL, "bad argument");
   if (!c->slot[0]) return fail(AMRVAC_FV_ESTATE, "no mesh");
   if (slot == 0 && c->dt_valid)
-    return getdt_reduce(c, courantpar, dtmin_out, cmax_out, c->d_dtp, c->n_dtp, c->d_red2);
+    return getdt_reduce(c, courantpar, dtmin_out, cmax_out, c->d_dtp, c->d_red2);
   return getdt_core(c, c->slot[slot], courantpar, dtmin_out, cmax_out, c->d_red, c->d_red2);
 }
 

@@ -115,6 +115,19 @@ __device__ __forceinline__ float fsqrt(float a) {
   else return __builtin_amdgcn_sqrtf(a);
 }
 
+// a / b for a divisor whose correctly rounded reciprocal is at hand: the
+// remainder of the rounded product corrects it to the correctly rounded
+// quotient (P. Markstein, IBM J. Res. Dev. 34, 1990), in 3 operations instead
+// of the 11 of the IEEE sequence
+__device__ __forceinline__ double div_by(double a, double b, double binv) {
+  if constexpr (kExact) {
+    return a / b;
+  } else {
+    const double q = a * binv;
+    return fma(fma(-q, b, a), binv, q);
+  }
+}
+
 // FP64 production arithmetic: the forms below that round differently from the
 // reference's expressions (by an ulp or two) are taken by these kernels only;
 // the bit-reproducible build and the FP32 faces keep the plain expressions.
@@ -297,7 +310,7 @@ __device__ __forceinline__ R fast_speed(const R* w, R gamma) {
 
 // hd_get_cbounds src/hd/mod_hd_phys.t:891-1001,
 // mhd_get_cbounds src/mhd/mod_mhd_phys.t:3037-3127
-template <class P, class R, int ID, bool WANT_CMIN>
+template <class P, class R, int ID, bool WANT_CMIN, bool PIN = false>
 __device__ __forceinline__ void cbounds(const R* wLC, const R* wRC, const R* wLp, const R* wRp,
                                         const FVParams& fp, R& cmax, R& cmin, int& crash) {
   const R g = R(fp.gamma);
@@ -391,9 +404,10 @@ __device__ __forceinline__ void cbounds(const R* wLC, const R* wRC, const R* wLp
       const R tmp1 = fsqrt(wLp[P::RHO]);
       const R tmp2 = fsqrt(wRp[P::RHO]);
       const R tmp3 = frcp(tmp1 + tmp2);
-      const R umean = (wLp[MN] * tmp1 + wRp[MN] * tmp2) * tmp3;
+      const R umean = (PIN ? fma(wLp[MN], tmp1, wRp[MN] * tmp2) : wLp[MN] * tmp1 + wRp[MN] * tmp2) * tmp3;
       const R dv = wRp[MN] - wLp[MN];
-      const R dmean = fsqrt((tmp1 * (csL * csL) + tmp2 * (csR * csR)) * tmp3 +
+      const R csq = PIN ? fma(tmp1, csL * csL, tmp2 * (csR * csR)) : tmp1 * (csL * csL) + tmp2 * (csR * csR);
+      const R dmean = fsqrt(csq * tmp3 +
                            R(0.5) * tmp1 * tmp2 * (tmp3 * tmp3) * (dv * dv));
       if constexpr (WANT_CMIN) {
         cmin = umean - dmean;
@@ -576,7 +590,9 @@ __device__ __forceinline__ void cada3_face32(const FVParams& fp, int id, R wm, R
 // WENO5limiter var=1 src/limiter/mod_weno.t:254-377, one variable, face
 // between cells 0 and 1 of the stencil s[-2..3] (passed as s0..s5 =
 // w(i-2)..w(i+3))
-template <class R>
+// PIN: 1 and 2 write out which of two products a multiply-add takes in, where
+// the compiler's choice depends on the code around the face (2: GLM's z faces)
+template <class R, int PIN = 0>
 __device__ __forceinline__ void weno5(R wmm, R wm, R w0, R wp, R wpp, R wppp, R& wl, R& wr) {
   const R bc1 = R(1.0833333333333333), bc2 = R(0.25);
   const R d1 = R(1.0 / 10.0), d2 = R(3.0 / 5.0), d3 = R(3.0 / 10.0);
@@ -586,34 +602,40 @@ __device__ __forceinline__ void weno5(R wmm, R wm, R w0, R wp, R wpp, R wppp, R&
   const R weps = R(1.0e-18);
   {
     const R f1 = u11 * wmm + u12 * wm + u13 * w0;
-    const R f2 = u21 * wm + u22 * w0 + u23 * wp;
-    const R f3 = u31 * w0 + u32 * wp + u33 * wpp;
+    const R f2 = PIN == 0   ? u21 * wm + u22 * w0 + u23 * wp
+                 : PIN == 1 ? fma(u23, wp, fma(u22, w0, u21 * wm))
+                            : fma(u23, wp, fma(u21, wm, u22 * w0));
+    const R f3 = PIN == 0 ? u31 * w0 + u32 * wp + u33 * wpp : fma(u33, wpp, fma(u31, w0, u32 * wp));
     R t = wmm + w0 - R(2) * wm, q = wmm - R(4) * wm + R(3) * w0;
     const R b1 = bc1 * (t * t) + bc2 * (q * q);
     t = wm + wp - R(2) * w0; q = wm - wp;
     const R b2 = bc1 * (t * t) + bc2 * (q * q);
     t = w0 + wpp - R(2) * wp; q = R(3) * w0 - R(4) * wp + wpp;
     const R b3 = bc1 * (t * t) + bc2 * (q * q);
-    t = b1 + weps; const R a1 = fdiv(d1, t * t);
-    t = b2 + weps; const R a2 = fdiv(d2, t * t);
-    t = b3 + weps; const R a3 = fdiv(d3, t * t);
-    const R as = a1 + a2 + a3;
+    t = b1 + weps; const R t1 = t * t, a1 = fdiv(d1, t1);
+    t = b2 + weps; const R t2 = t * t, a2 = fdiv(d2, t2);
+    t = b3 + weps; const R t3 = t * t, a3 = fdiv(d3, t3);
+    const R as = PIN == 0   ? a1 + a2 + a3
+                 : PIN == 1 ? fma(d3, frcp(t3), fma(d2, frcp(t2), a1))
+                            : fma(d3, frcp(t3), fma(d1, frcp(t1), a2));
     wl = fdiv(f1 * a1, as) + fdiv(f2 * a2, as) + fdiv(f3 * a3, as);
   }
   {
     const R f1 = u11 * wppp + u12 * wpp + u13 * wp;
-    const R f2 = u21 * wpp + u22 * wp + u23 * w0;
-    const R f3 = u31 * wp + u32 * w0 + u33 * wm;
+    const R f2 = PIN == 0 ? u21 * wpp + u22 * wp + u23 * w0 : fma(u23, w0, fma(u21, wpp, u22 * wp));
+    const R f3 = PIN == 0   ? u31 * wp + u32 * w0 + u33 * wm
+                 : PIN == 1 ? fma(u33, wm, fma(u32, w0, u31 * wp))
+                            : fma(u33, wm, fma(u31, wp, u32 * w0));
     R t = wppp + wp - R(2) * wpp, q = wppp - R(4) * wpp + R(3) * wp;
     const R b1 = bc1 * (t * t) + bc2 * (q * q);
     t = wpp + w0 - R(2) * wp; q = wpp - w0;
     const R b2 = bc1 * (t * t) + bc2 * (q * q);
     t = wp + wm - R(2) * w0; q = R(3) * wp - R(4) * w0 + wm;
     const R b3 = bc1 * (t * t) + bc2 * (q * q);
-    t = b1 + weps; const R a1 = fdiv(d1, t * t);
-    t = b2 + weps; const R a2 = fdiv(d2, t * t);
-    t = b3 + weps; const R a3 = fdiv(d3, t * t);
-    const R as = a1 + a2 + a3;
+    t = b1 + weps; const R t1 = t * t, a1 = fdiv(d1, t1);
+    t = b2 + weps; const R t2 = t * t, a2 = fdiv(d2, t2);
+    t = b3 + weps; const R t3 = t * t, a3 = fdiv(d3, t3);
+    const R as = PIN == 0 ? a1 + a2 + a3 : fma(d3, frcp(t3), fma(d2, frcp(t2), a1));
     wr = fdiv(f1 * a1, as) + fdiv(f2 * a2, as) + fdiv(f3 * a3, as);
   }
 }
@@ -797,7 +819,7 @@ struct CtIO {
   double cmax, cmin;
 };
 
-template <class P, class R, int RIEM, int ID, int LIM, int NG, bool CT = false>
+template <class P, class R, int RIEM, int ID, int LIM, int NG, bool CT = false, bool FIRST = false>
 __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& fp, R ch, R* fC,
                                           int& crash, CtIO* ctio = nullptr) {
   constexpr int NW = P::NW;
@@ -812,6 +834,9 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
       if constexpr (kFast64<R>)
         weno5_face64(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
                      tl[iw], tr[iw]);
+      else if (P::NDIM == 3 && std::is_same<R, float>::value && iw > 0)
+        weno5<R, P::GLM && ID == 2 && !FIRST ? 2 : 1>(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
+                       tl[iw], tr[iw]);
       else
         weno5(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
               tl[iw], tr[iw]);
@@ -902,12 +927,15 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
   phys_flux<P, R, ID>(wRC, wRp, ch, fR);
   R cmax, cmin = R(0);
   if constexpr (RIEM == RIEM_TVDLF) {
-    cbounds<P, R, ID, false>(wLC, wRC, wLp, wRp, fp, cmax, cmin, crash);
+    constexpr bool PIN = FIRST && LIM == LIM_WENO5 && !P::GLM && std::is_same<R, float>::value;
+    cbounds<P, R, ID, false, PIN>(wLC, wRC, wLp, wRp, fp, cmax, cmin, crash);
     if constexpr (CT) { ctio->cmax = cmax; ctio->cmin = cmin; }
     const R fac = R(-0.5) * R(fp.tvdlfeps) * cmax;
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) {
       fC[iw] = R(0.5) * (fL[iw] + fR[iw]);
+      if constexpr (FIRST && P::MHD && !(P::GLM && LIM == LIM_WENO5) && std::is_same<R, float>::value)
+        if (iw == P::RHO) fC[iw] = R(0.5) * fma(wLp[P::MOM + ID], wLp[P::RHO], fR[P::RHO]);
       fC[iw] = fC[iw] + fac * (wRC[iw] - wLC[iw]);
     }
   } else {

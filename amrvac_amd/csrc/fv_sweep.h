@@ -39,6 +39,7 @@ struct SweepArgs {
   int bnz;             // block_nx(3) (1 in 2-D)
   int per_xcd;         // ceil(nblocks/8)
   int zc;              // planes of a workgroup (3-D; bnz: the block is not split)
+  int src_al16;        // src is aligned to 16 bytes
   int comb_mode;       // 0: init = dst, 1: init = base, 2: init = a*base + b*src,
                        // 3: init = src (base is the stage input itself)
   double comb_a, comb_b;
@@ -181,8 +182,20 @@ __device__ __forceinline__ void load_prim(const SweepArgs& a, const FVParams& fp
 // The RK base and the output are touched once per launch: they stream
 // through L2 (non-temporal) so that they do not displace the stage input,
 // whose planes are re-read as halos by neighbouring workgroups.
-__device__ __forceinline__ double ld_stream(const double* p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ void st_stream(double v, double* p) { __builtin_nontemporal_store(v, p); }
+constexpr int kNonTemporal = 2;  // nt bit of the cache policy
+// bytes at p (the same for the whole wave) as a raw buffer
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_buffer(const double* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, bytes, 0x00020000);
+}
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+template <int POLICY>
+__device__ __forceinline__ double buffer_ld(__amdgpu_buffer_rsrc_t r, unsigned lane, unsigned off) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, lane, off, POLICY));
+}
+template <int POLICY>
+__device__ __forceinline__ void buffer_st(double v, __amdgpu_buffer_rsrc_t r, unsigned lane, unsigned off) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, v), r, lane, off, POLICY);
+}
 
 // Cell t of the four NG-deep halo strips of a plane (x and y block-local,
 // outside the block on one side), t < 4*NG*BX; then the 4 NG x NG corners.
@@ -203,6 +216,44 @@ __device__ __forceinline__ void strip_cell(int t, int& x, int& y) {
     x = (q & 1) ? BX + ox : -NG + ox;
     y = (q & 2) ? BX + oy : -NG + oy;
   }
+}
+
+// The halo strips of a plane as 16-byte pairs of neighbouring cells in x, 64
+// per variable of a 16^2 cross-section: pair p < 64 of the strips x-, x+ (16
+// rows), y-, y+ (2 rows of 8 pairs).  Offset of the pair's first cell in the
+// state, plane 0, variable 0; a physical boundary takes the cells of the
+// block that bc_phys mirrors or extends (which of the two, and the sign, is
+// the reader's: halo_elem).
+template <int NW>
+__device__ __forceinline__ size_t halo_pair(const SweepArgs& a, int b, int p) {
+  const int s = p >> 4, q = p & 15;
+  const int hi = s & 1, dim = s >> 1;
+  const int nbk = a.nbr[b * 27 + 13 + (hi ? 1 : -1) * (dim ? 3 : 1)];
+  const int depth = q >> 3;
+  int x, y;
+  if (dim == 0) {
+    y = q;
+    x = (nbk >= 0) == (hi != 0) ? 0 : 14;
+  } else {
+    x = 2 * (q & 7);
+    if (nbk >= 0) y = hi ? depth : 14 + depth;
+    else if (a.bc[2 + hi] == 2) y = hi ? 15 : 0;
+    else y = hi ? 15 - depth : 1 - depth;
+  }
+  const size_t cells = (size_t)256 * a.bnz;
+  return (size_t)(nbk >= 0 ? nbk : b) * NW * cells + y * 16 + x;
+}
+// Position (2 pair + element) of halo cell t < 128 (strip_cell's order) among
+// the pairs, and the sign of an antisymmetric boundary
+__device__ __forceinline__ int halo_elem(const SweepArgs& a, int b, int t, bool& neg) {
+  const int s = t >> 5, along = t & 15, depth = (t >> 4) & 1;
+  const int hi = s & 1, dim = s >> 1;
+  const bool phys = a.nbr[b * 27 + 13 + (hi ? 1 : -1) * (dim ? 3 : 1)] < 0;
+  const int bc = a.bc[2 * dim + hi];
+  neg = phys && bc == 4;
+  if (dim == 1) return 2 * (s * 16 + depth * 8 + (along >> 1)) + (along & 1);
+  const int e = !phys ? depth : (bc == 2 ? hi : 1 - depth);
+  return 2 * (s * 16 + along) + e;
 }
 
 // Occupancy: FP64 kernels run 2 waves per SIMD (LDS and registers), FP32
@@ -270,6 +321,9 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   __shared__ R fxs[HANCOCK ? 1 : NW][BX][BX + 1];  // x faces: fxs[iw][y][f]
   __shared__ R fys[HANCOCK ? 1 : NW][BX + 1][BX];  // y faces: fys[iw][f][x]
   __shared__ R hring[HRING ? NG : 1][HRING ? NW : 1][HRING ? NSTRIP : 1];
+  // the conserved halo pairs of the next plane, loaded straight into LDS
+  constexpr bool HPAIR = NDIM == 3 && !HRING && NG == 2 && BX == 16;
+  __shared__ __align__(16) double hraw[HPAIR ? NW : 1][HPAIR ? 128 : 1];
 
   const int b = wg_block(a.per_xcd);
   if (b >= a.nblocks) return;
@@ -297,7 +351,59 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   double dt_maxtot = -1.0e99, dt_cmax = 0.0;  // CFL partials of this lane's column
   const size_t cells = (size_t)BX * BX * a.bnz;
   const size_t boff = (size_t)b * NW * cells;
+  // Accesses to a block's planes in this lane's column: the block as a buffer
+  // in scalar registers, a scalar offset for plane and variable and this 32-bit
+  // lane offset, so that they take no vector address arithmetic.
+  const unsigned loff = 8u * (unsigned)(ty * BX + tx);
+  const unsigned vbytes = 8u * (unsigned)cells, bbytes = NW * vbytes;
+  auto block_ld = [&](const double* p, int k, double* c) {  // plane k of the block at p
+    const __amdgpu_buffer_rsrc_t r = block_buffer(p, bbytes);
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw) c[iw] = buffer_ld<0>(r, loff, k * (BX * BX * 8) + iw * vbytes);
+  };
+  auto block_ld_stream = [&](const double* p, int k, double* c) {
+    const __amdgpu_buffer_rsrc_t r = block_buffer(p, bbytes);
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw) c[iw] = buffer_ld<kNonTemporal>(r, loff, k * (BX * BX * 8) + iw * vbytes);
+  };
+  auto block_st_stream = [&](double* p, int k, const double* c) {
+    const __amdgpu_buffer_rsrc_t r = block_buffer(p, bbytes);
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw) buffer_st<kNonTemporal>(c[iw], r, loff, k * (BX * BX * 8) + iw * vbytes);
+  };
 
+  // lane's pair and halo cell
+  const double* hsrc = nullptr;
+  int hel = 0;
+  bool hneg = false;
+  if constexpr (HPAIR) {
+    hsrc = a.src + halo_pair<NW>(a, b, tid & 63);
+    hel = halo_elem(a, b, tid & 127, hneg);
+  }
+  // pairs of plane z into hraw: one 16-byte load per lane and variable; they
+  // are there after land_pairs and the barrier behind it.  A caller's array
+  // that is not aligned to 16 bytes is read in 8-byte loads.
+  auto load_pairs = [&](int z) {
+    if constexpr (HPAIR) {
+#pragma unroll
+      for (int i = 0; i < (NW + 3) / 4; ++i) {
+        const int iw = i * 4 + __builtin_amdgcn_readfirstlane(tid >> 6);
+        if (iw < NW) {
+          const double* p = hsrc + (size_t)z * BX * BX + iw * cells;
+          if (a.src_al16) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
+                                             (__attribute__((address_space(3))) void*)hraw[iw], 16, 0, 0);
+          } else {
+            hraw[iw][2 * (tid & 63)] = p[0];
+            hraw[iw][2 * (tid & 63) + 1] = p[1];
+          }
+        }
+      }
+    }
+  };
+  auto land_pairs = [&]() {
+    if constexpr (HPAIR) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  };
   const int nz = NDIM == 3 ? a.bnz : 1;
   const int z0 = NDIM == 3 ? (int)blockIdx.y * a.zc : 0;  // this workgroup's planes z0 .. z1-1
   const int z1 = NDIM == 3 ? (z0 + a.zc < nz ? z0 + a.zc : nz) : 1;
@@ -319,13 +425,48 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
     for (int m = 0; m < NG; ++m) prim_of<P, R>(Wc[m], Z[NG + m], fp);
   };
+  // the neighbours above and below are the same for all lanes
+  int nbz[2] = {0, 0};
+  if constexpr (NDIM == 3)
+#pragma unroll
+    for (int sd = 0; sd < 2; ++sd) nbz[sd] = __builtin_amdgcn_readfirstlane(a.nbr[b * 27 + 13 + (2 * sd - 1) * 9]);
+  // conserved plane z of this lane's column, z within NG of the block
+  // (locate for a cell outside the block in z alone)
+  auto load_plane = [&](int z, double* c) {
+    const double* pz = a.src + boff;
+    int zz = z;
+    bool neg = false;
+    if (z < 0 || z >= nz) {
+      const int sd = z < 0 ? 0 : 1;
+      const int nbk = sd ? nbz[1] : nbz[0];
+      if (nbk >= 0) {
+        pz = a.src + (size_t)nbk * NW * cells;
+        zz = sd ? z - nz : z + nz;
+      } else {
+        const int t = a.bc[4 + sd];
+        zz = t == 2 ? (sd ? nz - 1 : 0) : (sd ? 2 * nz - 1 - z : -1 - z);
+        neg = t == 4;
+      }
+    }
+    block_ld(pz, zz, c);
+    if (neg)
+#pragma unroll
+      for (int iw = 0; iw < NW; ++iw) c[iw] = -c[iw];
+  };
+  R zp[NW];  // primitive plane k+1, the next plane's own after it
   if constexpr (NDIM == 3) {
+    load_pairs(z0);
     // prologue: planes z0-NG .. z0+NG-1, halo ring of planes z0 .. z0+NG-1,
     // carried face z0-1/2
 #pragma unroll
-    for (int m = 0; m < NG; ++m) load_prim<P, R, NDIM, BX>(a, fp, b, tx, ty, z0 + m - NG, Wp[m]);
+    for (int m = 0; m < NG; ++m) {
+      double c[NW];
+      load_plane(z0 + m - NG, c);
+      prim_of<P, R>(c, Wp[m], fp);
+    }
 #pragma unroll
-    for (int m = 0; m < NG; ++m) load_cons_at<P, NDIM, BX>(a, b, tx, ty, z0 + m, Wc[m]);
+    for (int m = 0; m < NG; ++m) load_plane(z0 + m, Wc[m]);
+    prim_of<P, R>(Wc[0], zp, fp);
     if constexpr (HRING) {
       for (int p = z0; p < z0 + NG && p < z1; ++p)
         for (int t = tid; t < NSTRIP; t += NTHREADS) {
@@ -340,63 +481,19 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     if constexpr (!HANCOCK) {
       R Z[2 * NG][NW];
       zstencil(Z);
-      face_flux<P, R, RIEM, 2, LIM, NG>(Z, fp, ch, fz_carry, crash);
+      face_flux<P, R, RIEM, 2, LIM, NG, false, true>(Z, fp, ch, fz_carry, crash);
     }
-    if constexpr (HRING) __syncthreads();
+    land_pairs();
+    if constexpr (HRING || HPAIR) __syncthreads();
   }
 
-  for (int k = z0; k < z1; ++k) {
-    const size_t o = boff + ((size_t)k * BX + ty) * BX + tx;
-    double cons_k[NW];  // wCT of this lane's cell
-    double acc[NW];
-    // RK base (src/mod_advance.t:251-267), streamed; the combination with
-    // the stage input is formed once the base has arrived
-    auto rk_init = [&]() {
-      if (a.comb_mode == 0) {
+  // Plane k in LDS (primitive, with x/y halo); w: this lane's cell.  In 3-D the
+  // next plane is staged while this one's flux divergence is formed, which
+  // reads the face arrays and registers only: two barriers per plane.
+  auto stage_plane = [&](int k, const R* w) {
+    if (own)
 #pragma unroll
-        for (int iw = 0; iw < NW; ++iw) acc[iw] = ld_stream(a.dst + o + iw * cells);
-      } else if (a.comb_mode == 1) {
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) acc[iw] = ld_stream(a.base + o + iw * cells);
-      } else if (a.comb_mode == 2) {
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) acc[iw] = a.comb_a * ld_stream(a.base + o + iw * cells) + a.comb_b * cons_k[iw];
-      } else {
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) acc[iw] = cons_k[iw];
-      }
-    };
-    // ---- stage plane k (primitive, with x/y halo) in LDS -----------------
-    if constexpr (NDIM == 3) {
-      // advance the window and issue the lookahead plane k+NG
-#pragma unroll
-      for (int iw = 0; iw < NW; ++iw) cons_k[iw] = Wc[0][iw];
-      // fix_small_values: phys_to_primitive checks every cell it converts
-      // (src/hd/mod_hd_phys.t:713-715, src/mhd/mod_mhd_phys.t:1750-1753);
-      // over the level, the blocks' own cells are every converted cell
-      if (SMALLCHK && fp.fix_small && small_cons<P>(cons_k, fp)) crash = 1;
-#pragma unroll
-      for (int m = 0; m < NG - 1; ++m)
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) Wp[m][iw] = Wp[m + 1][iw];
-      prim_of<P, R>(cons_k, Wp[NG - 1], fp);
-#pragma unroll
-      for (int m = 0; m < NG - 1; ++m)
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) Wc[m][iw] = Wc[m + 1][iw];
-      load_cons_at<P, NDIM, BX>(a, b, tx, ty, k + NG, Wc[NG - 1]);
-      if (own)
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) sp[iw][ty + NG][tx + NG] = Wp[NG - 1][iw];
-    } else {
-      load_cons<P>(a.src, b, tx, ty, 0, BX, 1, cons_k);
-      if (SMALLCHK && fp.fix_small && small_cons<P>(cons_k, fp)) crash = 1;
-      R w[NW];
-      prim_of<P, R>(cons_k, w, fp);
-      if (own)
-#pragma unroll
-        for (int iw = 0; iw < NW; ++iw) sp[iw][ty + NG][tx + NG] = w[iw];
-    }
+      for (int iw = 0; iw < NW; ++iw) sp[iw][ty + NG][tx + NG] = w[iw];
     if constexpr (HRING) {
       const int slot = k % NG;
       for (int t = tid; t < NSTRIP; t += NTHREADS) {
@@ -404,6 +501,20 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
         strip_cell<NG, BX>(t, x, y);
 #pragma unroll
         for (int iw = 0; iw < NW; ++iw) sp[iw][y + NG][x + NG] = hring[slot][iw][t];
+      }
+    } else if constexpr (HPAIR) {
+      // halo strips of plane k from the pairs, by alternate wave pairs from
+      // plane to plane
+      if (((tid >> 7) ^ k) & 1) {
+        int x, y;
+        strip_cell<NG, BX>(tid & 127, x, y);
+        double c[NW];
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) c[iw] = hneg ? -hraw[iw][hel] : hraw[iw][hel];
+        R w[NW];
+        prim_of<P, R>(c, w, fp);
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) sp[iw][y + NG][x + NG] = w[iw];
       }
     } else {
       // halo strips of plane k (FP64: loaded by alternate wave pairs from
@@ -417,6 +528,59 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
         for (int iw = 0; iw < NW; ++iw) sp[iw][y + NG][x + NG] = w[iw];
       }
+    }
+  };
+  if constexpr (NDIM == 3) stage_plane(z0, zp);
+
+  for (int k = z0; k < z1; ++k) {
+    double cons_k[NW];  // wCT of this lane's cell
+    double acc[NW];
+    // RK base (src/mod_advance.t:251-267), streamed; the combination with
+    // the stage input is formed once the base has arrived
+    // (the production kernels fuse the stage input's product in 2-D and the
+    // base's in 3-D, whatever code surrounds the combination)
+    auto rk_init = [&]() {
+      if (a.comb_mode == 0) {
+        block_ld_stream(a.dst + boff, k, acc);
+      } else if (a.comb_mode == 1) {
+        block_ld_stream(a.base + boff, k, acc);
+      } else if (a.comb_mode == 2) {
+        block_ld_stream(a.base + boff, k, acc);
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw)
+          acc[iw] = kExact ? a.comb_a * acc[iw] + a.comb_b * cons_k[iw]
+                           : NDIM == 2 ? fma(a.comb_b, cons_k[iw], a.comb_a * acc[iw])
+                                       : fma(a.comb_a, acc[iw], a.comb_b * cons_k[iw]);
+      } else {
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) acc[iw] = cons_k[iw];
+      }
+    };
+    if constexpr (NDIM == 3) {
+      // advance the window and issue the lookahead plane k+NG
+#pragma unroll
+      for (int iw = 0; iw < NW; ++iw) cons_k[iw] = Wc[0][iw];
+      // fix_small_values: phys_to_primitive checks every cell it converts
+      // (src/hd/mod_hd_phys.t:713-715, src/mhd/mod_mhd_phys.t:1750-1753);
+      // over the level, the blocks' own cells are every converted cell
+      if (SMALLCHK && fp.fix_small && small_cons<P>(cons_k, fp)) crash = 1;
+#pragma unroll
+      for (int m = 0; m < NG - 1; ++m)
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) Wp[m][iw] = Wp[m + 1][iw];
+#pragma unroll
+      for (int iw = 0; iw < NW; ++iw) Wp[NG - 1][iw] = zp[iw];
+#pragma unroll
+      for (int m = 0; m < NG - 1; ++m)
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) Wc[m][iw] = Wc[m + 1][iw];
+      load_plane(k + NG, Wc[NG - 1]);
+    } else {
+      block_ld(a.src + boff, k, cons_k);
+      if (SMALLCHK && fp.fix_small && small_cons<P>(cons_k, fp)) crash = 1;
+      R w[NW];
+      prim_of<P, R>(cons_k, w, fp);
+      stage_plane(k, w);
     }
     __syncthreads();
     if constexpr (HRING) {
@@ -438,11 +602,28 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 
     // z neighbours of this lane's cell for the sources and the Hancock
     // predictor: primitive planes k-1 and k+1
-    R zm[NW], zp[NW];
+    R zm[NW];
     if constexpr (NDIM == 3) {
 #pragma unroll
       for (int iw = 0; iw < NW; ++iw) zm[iw] = Wp[NG - 2][iw];
     }
+    // extended GLM sources: the gradients of psi and B and the cell's own
+    // field, read from the plane before the next one takes its place
+    double glm_gp[2], glm_divb, glm_b[P::NDIR];
+    auto glm_gradients = [&]() {
+      if constexpr (P::GLM) {
+        constexpr int S = P::PSI;
+        const int cx = tx + NG, cy = ty + NG;
+        glm_gp[0] = div_by((double(sp[S][cy][cx + 1]) - double(sp[S][cy][cx - 1])) * 0.5, fp.dx[0], fp.dxinv[0]);
+        glm_gp[1] = div_by((double(sp[S][cy + 1][cx]) - double(sp[S][cy - 1][cx])) * 0.5, fp.dx[1], fp.dxinv[1]);
+        glm_divb = 0.0;
+        glm_divb = glm_divb + 0.5 * (double(sp[P::MAG][cy][cx + 1]) - double(sp[P::MAG][cy][cx - 1])) * fp.dxinv[0];
+        glm_divb =
+            glm_divb + 0.5 * (double(sp[P::MAG + 1][cy + 1][cx]) - double(sp[P::MAG + 1][cy - 1][cx])) * fp.dxinv[1];
+#pragma unroll
+        for (int d = 0; d < P::NDIR; ++d) glm_b[d] = double(sp[P::MAG + d][cy][cx]);
+      }
+    };
 
     if constexpr (!HANCOCK) {
       // ---- face fluxes of this plane --------------------------------------
@@ -479,6 +660,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
           for (int iw = 0; iw < NW; ++iw) fys[iw][f][x] = fc[iw];
         }
       }
+      if (HPAIR && k + 1 < z1) load_pairs(k + 1);
       rk_init();
       // z face k+1/2 last, so that the lookahead load has landed
       R fz_new[NW];
@@ -489,7 +671,10 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
         for (int iw = 0; iw < NW; ++iw) zp[iw] = Z[NG][iw];
       }
+      glm_gradients();
+      land_pairs();
       __syncthreads();
+      if (NDIM == 3 && k + 1 < z1) stage_plane(k + 1, zp);
       // ---- store_flux (src/mod_fix_conserve.t:597-648): the scaled fluxes
       //      of the block-boundary faces, for refluxing --------------------
       if (AMR && a.freg && own) {
@@ -522,6 +707,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       }
     } else {
       // ---- Hancock predictor (src/mod_finite_volume.t:19-113) -------------
+      if (HPAIR && k + 1 < z1) load_pairs(k + 1);
       rk_init();
       if constexpr (NDIM == 3) prim_of<P, R>(Wc[0], zp, fp);
       const R inv_g1 = R(fp.inv_gamma_1);
@@ -560,6 +746,12 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       }
       hancock_dim(std::integral_constant<int, 1>(), wm, w0, wp);
       if constexpr (NDIM == 3) hancock_dim(std::integral_constant<int, 2>(), zm, w0, zp);
+      glm_gradients();
+      land_pairs();
+      if constexpr (NDIM == 3) {
+        __syncthreads();
+        if (k + 1 < z1) stage_plane(k + 1, zp);
+      }
     }
 
     // ---- unphysical values after the flux update (finite_volume
@@ -577,19 +769,12 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       constexpr int S = P::PSI;
       acc[S] = glm_decay * acc[S];
       if (fp.glm_extended) {
-        const int cx = tx + NG, cy = ty + NG;
-        double gp[3], bn[3];
-        gp[0] = ((double(sp[S][cy][cx + 1]) - double(sp[S][cy][cx - 1])) * 0.5) / fp.dx[0];
-        gp[1] = ((double(sp[S][cy + 1][cx]) - double(sp[S][cy - 1][cx])) * 0.5) / fp.dx[1];
-        double divb = 0.0;
-        divb = divb + 0.5 * (double(sp[P::MAG][cy][cx + 1]) - double(sp[P::MAG][cy][cx - 1])) * fp.dxinv[0];
-        divb = divb + 0.5 * (double(sp[P::MAG + 1][cy + 1][cx]) - double(sp[P::MAG + 1][cy - 1][cx])) * fp.dxinv[1];
+        double gp[3] = {glm_gp[0], glm_gp[1], 0.0}, divb = glm_divb;
+        const double* bn = glm_b;
         if constexpr (NDIM == 3) {
-          gp[2] = ((double(zp[S]) - double(zm[S])) * 0.5) / fp.dx[2];
+          gp[2] = div_by((double(zp[S]) - double(zm[S])) * 0.5, fp.dx[2], fp.dxinv[2]);
           divb = divb + 0.5 * (double(zp[P::MAG + 2]) - double(zm[P::MAG + 2])) * fp.dxinv[2];
         }
-#pragma unroll
-        for (int d = 0; d < P::NDIR; ++d) bn[d] = double(sp[P::MAG + d][cy][cx]);
 #pragma unroll
         for (int d = 0; d < NDIM; ++d) acc[P::E] = acc[P::E] - a.qdt * bn[d] * gp[d];
 #pragma unroll
@@ -602,11 +787,9 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     if constexpr (P::GLM)
       if (SMALLCHK && fp.fix_small && small_cons<P>(acc, fp)) crash = 1;
     if (own)
-#pragma unroll
-      for (int iw = 0; iw < NW; ++iw) st_stream(acc[iw], a.dst + o + iw * cells);
+      block_st_stream(a.dst + boff, k, acc);
     if constexpr (CFL)
       if (a.dt_part) cfl_cell<P>(acc, fp, dt_maxtot, dt_cmax);
-    __syncthreads();  // LDS plane is rewritten next iteration
   }
   if (crash) *a.crash = 1;
   if constexpr (CFL) {
@@ -622,9 +805,8 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       if (tid == 0) {
         double m = dtr[0][0], c = dtr[1][0];
         for (int i = 1; i < NTHREADS / 64; ++i) { m = fmax(m, dtr[0][i]); c = fmax(c, dtr[1][i]); }
-        const int w = b * (int)gridDim.y + (int)blockIdx.y;
-        a.dt_part[2 * w] = m;
-        a.dt_part[2 * w + 1] = c;
+        a.dt_part[2 * b] = m;
+        a.dt_part[2 * b + 1] = c;
       }
     }
   }
