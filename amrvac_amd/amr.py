@@ -550,7 +550,7 @@ class AMRIntegrator(TimeIntegrator):
             regrid_due = self.ap.refine_max_level > 1 and (st.it + 1) % self.ap.ditregrid == 0
             flags = self.be.errest_flags(self.forest, self.ap) \
                 if regrid_due and getattr(self.be, "amr_device_regrid", False) else None
-            if st.crash or self.be.crash():
+            if st.crash or (getattr(self.be, "may_flag_small", True) and self.be.crash()):
                 st.crash = True
                 raise RuntimeError("Error: small value encountered, run crash.")
             if regrid_due:

@@ -35,14 +35,14 @@ constexpr double kSmall = 1.0e-12;  // src/mod_constants.t:8
 
 // Scratch of the allocation-free dt reduction (amrvac_fv_getdt_state_noalloc):
 // per-block partial maxima, 2 doubles per block for at most kNoallocMaxBlocks
-// blocks, then the reduced triple.  Every GPU the library runs on holds its
-// own copy (512 KiB) until the process ends.  In host code the array's name
-// is not a device address: kernels get the address hipGetSymbolAddress
-// returned for the context's device (amrvac_fv_ctx::scratch).
+// blocks.  Every GPU the library runs on holds its own copy (512 KiB) until the
+// process ends.  In host code the array's name is not a device address: kernels
+// get the address hipGetSymbolAddress returned for the context's device
+// (amrvac_fv_ctx::scratch).
 constexpr int kNoallocMaxBlocks = 32768;
 constexpr int kMaxDevices = 64;
 }  // namespace
-static __device__ __align__(256) double scratch[2 * kNoallocMaxBlocks + 4];
+static __device__ __align__(256) double scratch[2 * kNoallocMaxBlocks];
 namespace {
 double* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
@@ -93,7 +93,6 @@ struct amrvac_fv_ctx {
   double* d_dtp = nullptr;
   bool dt_valid = false;
   bool slot0_exposed = false;  // ps handed out by amrvac_fv_slot_pointer
-  double* d_red2 = nullptr;   // final reduction
   double* d_stage = nullptr;  // ghosted staging for download
   std::vector<double> h_stage;
   hipStream_t stream = nullptr;
@@ -136,9 +135,10 @@ struct amrvac_fv_ctx {
   std::vector<int> h_iws;     // the estimator's variables and weights as
   std::vector<double> h_wts;  // last uploaded
   // pinned host buffer of the results read back: the dt reduction's three
-  // doubles at 0, the small-value flag at kPinCrash, the regrid flags from
-  // kPinFlags followed (4-byte aligned) by the small-value flag copied with
-  // them (copies into it need no staging and share one synchronisation)
+  // doubles at 0, the small-value flag at kPinCrash, blocks' CFL maxima at
+  // kPinPart, the regrid flags from kPinFlags followed (4-byte aligned) by the small-value flag copied with
+  // them (copies and stores into it need no staging and share one
+  // synchronisation)
   char* h_pin = nullptr;
   size_t pin_cap = 0;
   int nrt = 0, npt = 0, nft = 0;
@@ -1153,7 +1153,11 @@ static bool ensure_buf(T** buf, size_t* cap, size_t n) {
   return true;
 }
 
-constexpr size_t kPinCrash = 24, kPinFlags = 32;
+// pinned buffer: the reduced CFL maxima and small-value flag (3 doubles), the
+// flag read by itself, the maxima of up to kPinBlocks blocks, then the
+// refinement flags
+constexpr int kPinBlocks = 1024;
+constexpr size_t kPinCrash = 24, kPinPart = 32, kPinFlags = kPinPart + kPinBlocks * 2 * sizeof(double);
 
 static bool ensure_pin(amrvac_fv_ctx* c, size_t bytes) {
   if (c->h_pin && c->pin_cap >= bytes) return true;
@@ -1169,8 +1173,17 @@ static bool ensure_pin(amrvac_fv_ctx* c, size_t bytes) {
   return true;
 }
 
+// whether any kernel of this configuration sets the small-value flag
+static bool may_flag_small(const amrvac_fv_ctx* c) {
+  return c->cfg.fix_small_values || (c->cfg.check_small_values && c->cfg.boundspeed == 2);
+}
+
 // the small-value flag, read back through the pinned buffer
 static hipError_t read_crash(amrvac_fv_ctx* c, int* out) {
+  if (!may_flag_small(c)) {
+    *out = 0;
+    return hipStreamSynchronize(c->stream);
+  }
   int* h = reinterpret_cast<int*>(c->h_pin + kPinCrash);
   hipError_t e = hipMemcpyAsync(h, c->d_crash, sizeof(int), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1271,12 +1284,11 @@ static void free_level(amrvac_fv_ctx* c) {
   if (c->d_nbr) (void)hipFree(c->d_nbr);
   if (c->d_crash) (void)hipFree(c->d_crash);
   if (c->d_red) (void)hipFree(c->d_red);
-  if (c->d_red2) (void)hipFree(c->d_red2);
   if (c->d_dtp) (void)hipFree(c->d_dtp);
   c->d_dtp = nullptr;
   c->dt_valid = false;
   if (c->d_stage) (void)hipFree(c->d_stage);
-  c->d_nbr = nullptr; c->d_crash = nullptr; c->d_red = nullptr; c->d_red2 = nullptr; c->d_stage = nullptr;
+  c->d_nbr = nullptr; c->d_crash = nullptr; c->d_red = nullptr; c->d_stage = nullptr;
   void* amr_bufs[] = {c->d_level, c->d_ntype, c->d_nchild, c->d_rtask, c->d_ptask, c->d_ptask2,
                       c->d_ftask, c->d_fregoff, c->d_freg, c->d_xlo, c->d_adjG};
   for (void* p : amr_bufs)
@@ -1414,7 +1426,7 @@ static int alloc_level(amrvac_fv_ctx* c, int nblocks, int capacity, const double
   if (!ensure_buf(&c->d_nbr, &c->nbr_cap, (size_t)nblocks * c->nnb) ||
       (!c->d_crash && hipMalloc(&c->d_crash, sizeof(int)) != hipSuccess) ||
       !ensure_buf(&c->d_red, &c->red_cap, (size_t)nblocks * 2 * (c->nw > 1 ? c->nw : 1)) ||
-      (!c->d_red2 && hipMalloc(&c->d_red2, sizeof(double) * 3) != hipSuccess) || !ensure_pin(c, kPinFlags + nblocks) ||
+      !ensure_pin(c, kPinFlags + nblocks) ||
       !ensure_buf(&c->d_dtp, &c->dtp_cap, (size_t)nblocks * 2) ||
       !ensure_buf(&c->d_stage, &c->stage_cap, (size_t)nblocks * c->nw * c->cells_g)) {
     free_level(c);
@@ -1552,38 +1564,55 @@ static int fix_conserve_amr(amrvac_fv_ctx* c, int slot) {
   return AMRVAC_FV_OK;
 }
 
-// reduction of the CFL maxima part[2*nb]: their max and the
-// small-value flag into fin[3], copied to the host; dt and cmax from them
-static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, double* cmax_out, double* part,
-                        double* fin);
-
-// dt of state u: per-block maxima into part[2*nb], then getdt_reduce
-static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, double* dtmin_out, double* cmax_out,
-                      double* part, double* fin) {
-  hipError_t e = with_phys<GetdtOp>(c, u, c->nb, c->bx, c->bnz, (const fvc::FVParams*)&c->fp, (const int*)c->d_level,
-                                    part, c->d_crash, c->stream);
-  if (e != hipSuccess) return fail(AMRVAC_FV_EHIP, std::string("getdt launch: ") + hipGetErrorString(e));
-  return getdt_reduce(c, courantpar, dtmin_out, cmax_out, part, fin);
+// dt and cmax from the maxima over the blocks
+static int dt_of_maxima(double m, double cm, double courantpar, double* dtmin_out, double* cmax_out) {
+  // min over blocks of courantpar/maxtot equals courantpar/max(maxtot): the
+  // correctly rounded quotient is monotone in the divisor
+  const double dt = m > kSmall ? courantpar / m : kBig;
+  if (dtmin_out) *dtmin_out = dt < kBig ? dt : kBig;
+  if (cmax_out) *cmax_out = cm;
+  return AMRVAC_FV_OK;
 }
 
-static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, double* cmax_out, double* part,
-                        double* fin) {
-  hipLaunchKernelGGL(fv::reduce_max2_kernel, dim3(1), dim3(fvc::NTHREADS), 0, c->stream, part, c->nb, fin,
-                     (const int*)c->d_crash);
-  HIPCHK(hipGetLastError());
+// reduction of the CFL maxima part[2*nb]: their max and the small-value flag,
+// written to the pinned buffer by the kernel; dt and cmax from them
+static int getdt_reduce(amrvac_fv_ctx* c, double courantpar, double* dtmin_out, double* cmax_out,
+                        const double* part) {
   const double* r = reinterpret_cast<const double*>(c->h_pin);
-  HIPCHK(hipMemcpyAsync(c->h_pin, fin, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  hipLaunchKernelGGL(fv::reduce_max2_kernel, dim3(1), dim3(fvc::NTHREADS), 0, c->stream, part, c->nb,
+                     reinterpret_cast<double*>(c->h_pin), (const int*)c->d_crash);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->stream));
   // the small-value flag as of this reduction; valid until the next launch
   // that may set it
   c->crash_seen = r[2] != 0.0 ? 1 : 0;
   c->crash_fresh = true;
-  // min over blocks of courantpar/maxtot equals courantpar/max(maxtot): the
-  // correctly rounded quotient is monotone in the divisor
-  const double dt = r[0] > kSmall ? courantpar / r[0] : kBig;
-  if (dtmin_out) *dtmin_out = dt < kBig ? dt : kBig;
-  if (cmax_out) *cmax_out = r[1];
-  return AMRVAC_FV_OK;
+  return dt_of_maxima(r[0], r[1], courantpar, dtmin_out, cmax_out);
+}
+
+// dt of state u: per-block maxima, then their reduction.  Where no kernel sets
+// the small-value flag the maxima of up to kPinBlocks blocks go straight to the
+// pinned buffer and are reduced here: the time is then that of the launches and
+// the wait, and this takes one launch instead of two and a copy (256^2 HD, 256
+// blocks: a step 58 -> 41 us with the small-value flag's wait left out).  More
+// blocks leave the host more to read than a second launch costs.
+static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, double* dtmin_out, double* cmax_out,
+                      double* part) {
+  const bool pin = c->nb <= kPinBlocks && !may_flag_small(c);
+  double* out = pin ? reinterpret_cast<double*>(c->h_pin + kPinPart) : part;
+  hipError_t e = with_phys<GetdtOp>(c, u, c->nb, c->bx, c->bnz, (const fvc::FVParams*)&c->fp, (const int*)c->d_level,
+                                    out, c->d_crash, c->stream);
+  if (e != hipSuccess) return fail(AMRVAC_FV_EHIP, std::string("getdt launch: ") + hipGetErrorString(e));
+  if (!pin) return getdt_reduce(c, courantpar, dtmin_out, cmax_out, part);
+  HIPCHK(hipStreamSynchronize(c->stream));
+  c->crash_seen = 0;
+  c->crash_fresh = true;
+  double m = -1.0e99, cm = 0.0;
+  for (int b = 0; b < c->nb; ++b) {
+    m = std::fmax(m, out[2 * b]);
+    cm = std::fmax(cm, out[2 * b + 1]);
+  }
+  return dt_of_maxima(m, cm, courantpar, dtmin_out, cmax_out);
 }
 
 // Planes per workgroup of a 3-D stage.  One workgroup marches through its
@@ -1851,8 +1880,8 @@ int amrvac_fv_getdt(amrvac_fv_ctx* c, int slot, double courantpar, double* dtmin
   if (!c || !check_slot(slot)) return fail(AMRVAC_FV_EINVAL, "bad argument");
   if (!c->slot[0]) return fail(AMRVAC_FV_ESTATE, "no mesh");
   if (slot == 0 && c->dt_valid)
-    return getdt_reduce(c, courantpar, dtmin_out, cmax_out, c->d_dtp, c->d_red2);
-  return getdt_core(c, c->slot[slot], courantpar, dtmin_out, cmax_out, c->d_red, c->d_red2);
+    return getdt_reduce(c, courantpar, dtmin_out, cmax_out, c->d_dtp);
+  return getdt_core(c, c->slot[slot], courantpar, dtmin_out, cmax_out, c->d_red);
 }
 
 int amrvac_fv_getdt_state(amrvac_fv_ctx* c, const double* u, double courantpar, double* dtmin_out,
@@ -1860,7 +1889,7 @@ int amrvac_fv_getdt_state(amrvac_fv_ctx* c, const double* u, double courantpar, 
   if (!c || !u) return fail(AMRVAC_FV_EINVAL, "bad argument");
   if (!c->slot[0]) return fail(AMRVAC_FV_ESTATE, "no mesh");
   if (c->amr) return fail(AMRVAC_FV_EINVAL, "state arrays are for a uniform level");
-  return getdt_core(c, u, courantpar, dtmin_out, cmax_out, c->d_red, c->d_red2);
+  return getdt_core(c, u, courantpar, dtmin_out, cmax_out, c->d_red);
 }
 
 int amrvac_fv_getdt_state_noalloc(amrvac_fv_ctx* c, const double* u, double courantpar, double* dtmin_out,
@@ -1872,9 +1901,9 @@ int amrvac_fv_getdt_state_noalloc(amrvac_fv_ctx* c, const double* u, double cour
     return fail(AMRVAC_FV_EINVAL, "amrvac_fv_getdt_state_noalloc takes at most 32768 blocks "
                                   "(its scratch array holds two partial maxima per block)");
   if (!c->scratch) return fail(AMRVAC_FV_ESTATE, "no scratch address for this device");
-  // every per-block entry and the reduced triple are overwritten: nothing
-  // in the scratch needs clearing between calls
-  return getdt_core(c, u, courantpar, dtmin_out, cmax_out, c->scratch, c->scratch + 2 * kNoallocMaxBlocks);
+  // every per-block entry is overwritten: nothing in the scratch needs
+  // clearing between calls
+  return getdt_core(c, u, courantpar, dtmin_out, cmax_out, c->scratch);
 }
 
 int amrvac_fv_advect1(amrvac_fv_ctx* c, int method, double dtfactor, double dt, double cmax_global, int psa,

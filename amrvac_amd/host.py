@@ -18,6 +18,8 @@ Backend protocol (slots 0=ps, 1=ps1, 2=ps2, 3=ps3):
                                   slots (see Expr), one rounding per node
   volume_average(slot) -> ndarray[2*nw]
   crash() -> bool
+  may_flag_small (optional, default True)
+      False: no operation of this configuration raises the crash flag
 """
 from __future__ import annotations
 
@@ -460,7 +462,9 @@ class TimeIntegrator:
             self.advect()
             st.dts.append(st.dt)
             st.chs.append(st.cmax_global)
-            if st.crash or self.be.crash():
+            # a configuration whose kernels never set the flag need not wait
+            # for it here: the next setdt waits for the stages
+            if st.crash or (getattr(self.be, "may_flag_small", True) and self.be.crash()):
                 st.crash = True
                 raise RuntimeError("Error: small value encountered, run crash.")
             st.it += 1
