@@ -1790,6 +1790,8 @@ static int ct_stage(amrvac_fv_ctx* c, int method, double dtfactor, double dt, in
   a.comb_b = comb_b;
   const double qdt = dtfactor * dt;
   a.qdt = qdt;
+  a.zc = stage_zc(c);
+  a.src_al16 = reinterpret_cast<uintptr_t>(a.src) % 16 == 0;
   for (int d = 0; d < 3; ++d) a.dq[d] = -qdt / c->dx[d];
   c->crash_fresh = false;
   if (psb == 0) c->dt_valid = false;

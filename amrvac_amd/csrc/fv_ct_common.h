@@ -21,8 +21,8 @@ struct CtArgs {
   int ct;                  // CT_*
   int tgc;                 // transverse_ghost_cells
   int tvdlf;               // 1: no cmin (cbarmin = cbarmax)
-  // 3-D scratch (per block, cells -2..17 in each direction)
-  void* prim;              // primitive state, face precision
+  // 3-D scratch
+  double* data;            // face data of the edge fields
   double* ecc;             // b x v at cell centres (uct_contact)
   double* edges;           // edge electric fields times qdt and edge length
 };

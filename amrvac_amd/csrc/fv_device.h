@@ -261,7 +261,9 @@ __device__ __forceinline__ void to_cons(R* w, R inv_gamma_1) {
 
 // hd_get_flux src/hd/mod_hd_phys.t:1097-1146,
 // mhd_get_flux src/mhd/mod_mhd_phys.t:3810-3889 (GLM :3868-3874)
-template <class P, class R, int ID>
+// PIN_BN: in b.v the normal field's product is not the fused one whatever code
+// surrounds the flux
+template <class P, class R, int ID, bool PIN_BN = false>
 __device__ __forceinline__ void phys_flux(const R* wC, const R* w, R ch, R* f) {
   const R vn = w[P::MOM + ID];
   if constexpr (!P::MHD) {
@@ -281,8 +283,15 @@ __device__ __forceinline__ void phys_flux(const R* wC, const R* w, R ch, R* f) {
     const R ptotal = w[P::E] + R(0.5) * bsq;
     f[P::MOM + ID] = f[P::MOM + ID] + ptotal;
     R bv = w[P::MAG] * w[P::MOM];
+    if constexpr (PIN_BN && ID < 2) {
+      constexpr int O = 1 - ID;
+      bv = fma(w[P::MAG + O], w[P::MOM + O], bn * vn);
 #pragma unroll
-    for (int d = 1; d < P::NDIR; ++d) bv = bv + w[P::MAG + d] * w[P::MOM + d];
+      for (int d = 2; d < P::NDIR; ++d) bv = fma(w[P::MAG + d], w[P::MOM + d], bv);
+    } else {
+#pragma unroll
+      for (int d = 1; d < P::NDIR; ++d) bv = bv + w[P::MAG + d] * w[P::MOM + d];
+    }
     f[P::E] = vn * (wC[P::E] + ptotal) - bn * bv;
 #pragma unroll
     for (int d = 0; d < P::NDIR; ++d) f[P::MAG + d] = vn * w[P::MAG + d] - bn * w[P::MOM + d];
@@ -891,7 +900,7 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
   }
 #pragma unroll
   for (int iw = 0; iw < NW; ++iw) { wLC[iw] = wLp[iw]; wRC[iw] = wRp[iw]; }
-  constexpr bool FUSE_P = LIM == LIM_CADA3 && std::is_same<R, float>::value;
+  constexpr bool FUSE_P = (CT || LIM == LIM_CADA3) && std::is_same<R, float>::value;
   to_cons<P, R, FUSE_P>(wLC, inv_g1);
   to_cons<P, R, FUSE_P>(wRC, inv_g1);
   if constexpr (P::GLM && !GLM_FIRST) {
@@ -923,8 +932,9 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
     }
   }
   R fL[NW], fR[NW];
-  phys_flux<P, R, ID>(wLC, wLp, ch, fL);
-  phys_flux<P, R, ID>(wRC, wRp, ch, fR);
+  constexpr bool PIN_BN = CT && P::NDIM == 3 && (LIM == LIM_MINMOD || LIM == LIM_VANLEER) && std::is_same<R, float>::value;
+  phys_flux<P, R, ID, PIN_BN>(wLC, wLp, ch, fL);
+  phys_flux<P, R, ID, PIN_BN>(wRC, wRp, ch, fR);
   R cmax, cmin = R(0);
   if constexpr (RIEM == RIEM_TVDLF) {
     constexpr bool PIN = FIRST && LIM == LIM_WENO5 && !P::GLM && std::is_same<R, float>::value;
@@ -934,7 +944,7 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) {
       fC[iw] = R(0.5) * (fL[iw] + fR[iw]);
-      if constexpr (FIRST && P::MHD && !(P::GLM && LIM == LIM_WENO5) && std::is_same<R, float>::value)
+      if constexpr ((FIRST || CT) && P::MHD && !(P::GLM && LIM == LIM_WENO5) && std::is_same<R, float>::value)
         if (iw == P::RHO) fC[iw] = R(0.5) * fma(wLp[P::MOM + ID], wLp[P::RHO], fR[P::RHO]);
       fC[iw] = fC[iw] + fac * (wRC[iw] - wLC[iw]);
     }

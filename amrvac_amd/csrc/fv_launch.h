@@ -85,10 +85,10 @@ template <class P, class R, int RIEM, int LIM, int NG>
 hipError_t launch_one(const SweepArgs& a, const FVParams& fp, int grid, hipStream_t s) {
   if (a.blevel)
     hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, true, 16>), sweep_grid(a, grid), dim3(kLanes<16>), 0, s, a,
-                       fp);
+                       fp, NoCt{});
   else
     hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, LIM, NG, false, 16>), sweep_grid(a, grid), dim3(kLanes<16>), 0, s, a,
-                       fp);
+                       fp, NoCt{});
   return hipGetLastError();
 }
 
@@ -98,7 +98,7 @@ hipError_t launch_one(const SweepArgs& a, const FVParams& fp, int grid, hipStrea
 template <class P, class R, int RIEM, int NG, int BXc>
 hipError_t launch_small(const SweepArgs& a, const FVParams& fp, int grid, hipStream_t s) {
   hipLaunchKernelGGL((sweep_kernel<P, R, RIEM, NG == 3 ? LIM_WENO5 : 0, NG, true, BXc>), sweep_grid(a, grid),
-                     dim3(kLanes<BXc>), 0, s, a, fp);
+                     dim3(kLanes<BXc>), 0, s, a, fp, NoCt{});
   return hipGetLastError();
 }
 

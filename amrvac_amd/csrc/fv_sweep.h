@@ -286,12 +286,18 @@ __device__ __forceinline__ void level_params(const SweepArgs& a, int b, FVParams
   glm_decay = a.glm_decay_lev[lev];
 }
 
+// Cell-centred field: nothing beside the flux update
+struct NoCt {};
+
 // AMR: level-dependent scheme constants and the refluxing registers; the
 // uniform-level kernels are compiled without them (their registers would
 // spill in the 3-D MHD kernels).
-template <class P, class R, int RIEM, int LIM, int NG, bool AMR, int BXc>
+// CTA: a 3-D stage of constrained transport (its face field, face data and
+// edge fields; fv_ct3.hip): the faces take their normal field from it and give
+// it what the edge fields need, and the update leaves out the field.
+template <class P, class R, int RIEM, int LIM, int NG, bool AMR, int BXc, class CTA = NoCt>
 __global__ void __launch_bounds__(kLanes<BXc>, kMinWaves<R>)
-sweep_kernel(SweepArgs a, FVParams fp0) {
+sweep_kernel(SweepArgs a, FVParams fp0, CTA ct) {
   constexpr int BX = BXc;                 // block_nx(1) = block_nx(2)
   constexpr int NTHREADS = kLanes<BXc>;   // lanes of the workgroup
   constexpr bool FULL = BX * BX == NTHREADS;
@@ -299,6 +305,8 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   constexpr int NW = P::NW;
   constexpr int PX = BX + 2 * NG;
   constexpr bool HANCOCK = RIEM == RIEM_HANCOCK;
+  constexpr bool CT = !std::is_same<CTA, NoCt>::value;
+  constexpr int NF = CT ? P::MAG : NW;    // variables updated from their fluxes
   // Any extra runtime branch in the z loop of the specialised kernels (a
   // compile-time TVD limiter on a uniform level of 16^2 cross-sections)
   // costs the FP64 form about 12% (measured): they carry no small-value
@@ -306,8 +314,8 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   // and only the FP32-reconstruction form, where the fused CFL partials cost
   // 2% and save the separate pass over ps, computes them.
   constexpr bool SPECIAL = LIM != 0 && LIM != LIM_WENO5 && !AMR && BXc == 16;
-  constexpr bool SMALLCHK = !SPECIAL;
-  constexpr bool CFL = !AMR && BXc == 16 && std::is_same<R, float>::value;
+  constexpr bool SMALLCHK = !SPECIAL && !CT;
+  constexpr bool CFL = !AMR && !CT && BXc == 16 && std::is_same<R, float>::value;
   constexpr int NSTRIP = 4 * NG * BX;
   constexpr int NHALO = NSTRIP;
   // 3-D, FP32 reconstruction: the halo strips of the NG planes ahead are
@@ -318,8 +326,8 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   constexpr bool HRING = NDIM == 3 && std::is_same<R, float>::value;
 
   __shared__ R sp[NW][PX][PX];          // primitive plane with halo
-  __shared__ R fxs[HANCOCK ? 1 : NW][BX][BX + 1];  // x faces: fxs[iw][y][f]
-  __shared__ R fys[HANCOCK ? 1 : NW][BX + 1][BX];  // y faces: fys[iw][f][x]
+  __shared__ R fxs[HANCOCK ? 1 : NF][BX][BX + 1];  // x faces: fxs[iw][y][f]
+  __shared__ R fys[HANCOCK ? 1 : NF][BX + 1][BX];  // y faces: fys[iw][f][x]
   __shared__ R hring[HRING ? NG : 1][HRING ? NW : 1][HRING ? NSTRIP : 1];
   // the conserved halo pairs of the next plane, loaded straight into LDS
   constexpr bool HPAIR = NDIM == 3 && !HRING && NG == 2 && BX == 16;
@@ -327,6 +335,11 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 
   const int b = wg_block(a.per_xcd);
   if (b >= a.nblocks) return;
+  __shared__ int nbs[CT ? 27 : 1];        // the block's neighbours (CT)
+  if constexpr (CT) {
+    if (threadIdx.x < 27) nbs[threadIdx.x] = a.nbr[b * 27 + threadIdx.x];
+    __syncthreads();
+  }
   FVParams fp = fp0;
   double dq[3], glm_decay;
   // refluxing registers of the block's faces (x-, x+, y-, y+, z-, z+)
@@ -364,12 +377,12 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
   auto block_ld_stream = [&](const double* p, int k, double* c) {
     const __amdgpu_buffer_rsrc_t r = block_buffer(p, bbytes);
 #pragma unroll
-    for (int iw = 0; iw < NW; ++iw) c[iw] = buffer_ld<kNonTemporal>(r, loff, k * (BX * BX * 8) + iw * vbytes);
+    for (int iw = 0; iw < NF; ++iw) c[iw] = buffer_ld<kNonTemporal>(r, loff, k * (BX * BX * 8) + iw * vbytes);
   };
   auto block_st_stream = [&](double* p, int k, const double* c) {
     const __amdgpu_buffer_rsrc_t r = block_buffer(p, bbytes);
 #pragma unroll
-    for (int iw = 0; iw < NW; ++iw) buffer_st<kNonTemporal>(c[iw], r, loff, k * (BX * BX * 8) + iw * vbytes);
+    for (int iw = 0; iw < NF; ++iw) buffer_st<kNonTemporal>(c[iw], r, loff, k * (BX * BX * 8) + iw * vbytes);
   };
 
   // lane's pair and halo cell
@@ -481,7 +494,9 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
     if constexpr (!HANCOCK) {
       R Z[2 * NG][NW];
       zstencil(Z);
-      face_flux<P, R, RIEM, 2, LIM, NG, false, true>(Z, fp, ch, fz_carry, crash);
+      [[maybe_unused]] CtIO io;
+      if constexpr (CT) ct.template face_in<RIEM, 2>(a, io, nbs, tx, ty, z0 - 1);
+      face_flux<P, R, RIEM, 2, LIM, NG, CT, true>(Z, fp, ch, fz_carry, crash, &io);
     }
     land_pairs();
     if constexpr (HRING || HPAIR) __syncthreads();
@@ -547,13 +562,13 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       } else if (a.comb_mode == 2) {
         block_ld_stream(a.base + boff, k, acc);
 #pragma unroll
-        for (int iw = 0; iw < NW; ++iw)
+        for (int iw = 0; iw < NF; ++iw)
           acc[iw] = kExact ? a.comb_a * acc[iw] + a.comb_b * cons_k[iw]
                            : NDIM == 2 ? fma(a.comb_b, cons_k[iw], a.comb_a * acc[iw])
                                        : fma(a.comb_a, acc[iw], a.comb_b * cons_k[iw]);
       } else {
 #pragma unroll
-        for (int iw = 0; iw < NW; ++iw) acc[iw] = cons_k[iw];
+        for (int iw = 0; iw < NF; ++iw) acc[iw] = cons_k[iw];
       }
     };
     if constexpr (NDIM == 3) {
@@ -575,6 +590,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
         for (int iw = 0; iw < NW; ++iw) Wc[m][iw] = Wc[m + 1][iw];
       load_plane(k + NG, Wc[NG - 1]);
+      if constexpr (CT) ct.template cell_out<P, R>(fp, cons_k, Wp[NG - 1], b, tx, ty, k);
     } else {
       block_ld(a.src + boff, k, cons_k);
       if (SMALLCHK && fp.fix_small && small_cons<P>(cons_k, fp)) crash = 1;
@@ -643,9 +659,13 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
             for (int iw = 0; iw < NW; ++iw) st[s][iw] = sp[iw][y + NG][f + s];
           R fc[NW];
-          face_flux<P, R, RIEM, 0, LIM, NG>(st, fp, ch, fc, crash);
+          [[maybe_unused]] CtIO io;
+          if constexpr (CT) ct.template face_in<RIEM, 0>(a, io, nbs, f - 1, y, k);
+          face_flux<P, R, RIEM, 0, LIM, NG, CT>(st, fp, ch, fc, crash, &io);
+          if constexpr (CT)
+            if (f > 0) ct.template face_out<P, R, 0>(io, fc, b, f - 1, y, k);
 #pragma unroll
-          for (int iw = 0; iw < NW; ++iw) fxs[iw][y][f] = fc[iw];
+          for (int iw = 0; iw < NF; ++iw) fxs[iw][y][f] = fc[iw];
         } else if (t >= XSLOTS) {
           const int u = t - XSLOTS;
           const int f = u / BX, x = u % BX;  // face between f-1 and f
@@ -655,9 +675,13 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
 #pragma unroll
             for (int iw = 0; iw < NW; ++iw) st[s][iw] = sp[iw][f + s][x + NG];
           R fc[NW];
-          face_flux<P, R, RIEM, 1, LIM, NG>(st, fp, ch, fc, crash);
+          [[maybe_unused]] CtIO io;
+          if constexpr (CT) ct.template face_in<RIEM, 1>(a, io, nbs, x, f - 1, k);
+          face_flux<P, R, RIEM, 1, LIM, NG, CT>(st, fp, ch, fc, crash, &io);
+          if constexpr (CT)
+            if (f > 0) ct.template face_out<P, R, 1>(io, fc, b, x, f - 1, k);
 #pragma unroll
-          for (int iw = 0; iw < NW; ++iw) fys[iw][f][x] = fc[iw];
+          for (int iw = 0; iw < NF; ++iw) fys[iw][f][x] = fc[iw];
         }
       }
       if (HPAIR && k + 1 < z1) load_pairs(k + 1);
@@ -667,7 +691,10 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       if constexpr (NDIM == 3) {
         R Z[2 * NG][NW];
         zstencil(Z);
-        face_flux<P, R, RIEM, 2, LIM, NG>(Z, fp, ch, fz_new, crash);
+        [[maybe_unused]] CtIO io;
+        if constexpr (CT) ct.template face_in<RIEM, 2>(a, io, nbs, tx, ty, k);
+        face_flux<P, R, RIEM, 2, LIM, NG, CT>(Z, fp, ch, fz_new, crash, &io);
+        if constexpr (CT) ct.template face_out<P, R, 2>(io, fz_new, b, tx, ty, k);
 #pragma unroll
         for (int iw = 0; iw < NW; ++iw) zp[iw] = Z[NG][iw];
       }
@@ -697,7 +724,7 @@ sweep_kernel(SweepArgs a, FVParams fp0) {
       }
       // ---- flux divergence, dimension by dimension (:269-284) ------------
 #pragma unroll
-      for (int iw = 0; iw < NW; ++iw) {
+      for (int iw = 0; iw < NF; ++iw) {
         acc[iw] = acc[iw] + dq[0] * double(fxs[iw][ty][tx + 1]) - dq[0] * double(fxs[iw][ty][tx]);
         acc[iw] = acc[iw] + dq[1] * double(fys[iw][ty + 1][tx]) - dq[1] * double(fys[iw][ty][tx]);
         if constexpr (NDIM == 3) {
