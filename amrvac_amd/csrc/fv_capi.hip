@@ -681,8 +681,12 @@ __device__ __forceinline__ double cell_value(const SweepArgs& a, int nw, int b, 
 // Built without contraction, so every build rounds like the oracle.
 // Bound by address arithmetic and the latency of the lookups (six field values
 // per rim cell): the cross-section is a compile-time constant and the block's
-// neighbours are read into LDS once (3186 blocks of 8^3: 142 to 120 us).
-constexpr int kLindeLds = 7800;  // doubles: (bx+2)^2 (bnz+2) for bx <= 16, bnz <= 22
+// neighbours are read into LDS once; LDS for the block's own size lets a CU hold
+// more blocks (3186 blocks of 8^3: 142, then 120, then 85 us).
+constexpr int kLindeLds = 7800;  // doubles at most: (bx+2)^2 (bnz+2) for bx <= 16, bnz <= 22
+inline size_t linde_lds(int ndim, int bx, int bnz) {
+  return (size_t)(bx + 2) * (bx + 2) * (ndim == 3 ? bnz + 2 : 1) * sizeof(double);
+}
 template <class P, int bx>
 __global__ void __launch_bounds__(NTHREADS) linde_kernel(SweepArgs a, FVParams fp, const int* __restrict__ ntype,
                                                          int nnb, double* __restrict__ dst) {
@@ -701,7 +705,7 @@ __global__ void __launch_bounds__(NTHREADS) linde_kernel(SweepArgs a, FVParams f
   const int bz = NDIM == 3 ? a.bnz : 1;
   constexpr int ex = bx + 2;
   const int ez = NDIM == 3 ? bz + 2 : 1;
-  __shared__ double divb[kLindeLds];
+  extern __shared__ double divb[];
   __shared__ int nbrs[NNB];
   if (threadIdx.x < NNB) nbrs[threadIdx.x] = a.nbr[(size_t)b * NNB + threadIdx.x];
   __syncthreads();
@@ -773,13 +777,14 @@ hipError_t launch_linde(const SweepArgs& a, const FVParams& fp, const int* ntype
   if constexpr (!P::MHD || P::NDIM < 2) {
     return hipErrorInvalidValue;
   } else {
+    const size_t lds = linde_lds(P::NDIM, a.bx, a.bnz);
     if (a.bx == 16) {
-      hipLaunchKernelGGL((linde_kernel<P, 16>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+      hipLaunchKernelGGL((linde_kernel<P, 16>), dim3(a.nblocks), dim3(NTHREADS), lds, s, a, fp, ntype, nnb, dst);
     } else if constexpr (P::NDIM == 3) {
       if (a.bx == 8)
-        hipLaunchKernelGGL((linde_kernel<P, 8>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+        hipLaunchKernelGGL((linde_kernel<P, 8>), dim3(a.nblocks), dim3(NTHREADS), lds, s, a, fp, ntype, nnb, dst);
       else if (a.bx == 10)
-        hipLaunchKernelGGL((linde_kernel<P, 10>), dim3(a.nblocks), dim3(NTHREADS), 0, s, a, fp, ntype, nnb, dst);
+        hipLaunchKernelGGL((linde_kernel<P, 10>), dim3(a.nblocks), dim3(NTHREADS), lds, s, a, fp, ntype, nnb, dst);
       else
         return hipErrorInvalidValue;
     } else {
