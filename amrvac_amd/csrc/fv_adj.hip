@@ -36,16 +36,32 @@ constexpr int NF = BX + 3;        // faces per row touching the tile: f in [-1, 
 constexpr int NFACE = NF * BX;    // per dimension and plane
 constexpr int ZC = 16;            // cells per lane and chunk in adj_zface_kernel
 
-// lam_out at an arbitrary (possibly neighbouring) cell of plane z
-template <int NW, int NDIM>
-__device__ __forceinline__ void load_lam(const SweepArgs& a, const double* __restrict__ lam, int b, int x, int y,
-                                         int z, double* l) {
-  double sign;
-  const int sb = locate<NDIM>(a, b, x, y, z, sign);
-  const size_t cells = (size_t)BX * BX * a.bnz;
-  const size_t off = (size_t)sb * NW * cells + ((size_t)z * BX + y) * BX + x;
+// the NW values of w at offset off of variable 0
+template <int NW>
+__device__ __forceinline__ void load_at(const double* __restrict__ w, size_t off, size_t cells, double* c) {
 #pragma unroll
-  for (int iw = 0; iw < NW; ++iw) l[iw] = lam[off + iw * cells];
+  for (int iw = 0; iw < NW; ++iw) c[iw] = w[off + iw * cells];
+}
+
+// Variable 0 of a cell of the block's plane k or beside it in x or y.  nbs: the
+// plane's 9 neighbours in LDS (the level is periodic: all exist), so that the
+// staging waits for one look into the level's table, not for one per value
+// (128^3 MHD-GLM, FP32 faces: plane kernel 342 -> 314 us, 309 with both rounds
+// of the tiles in flight; 128^2 HD: 12.5 -> 11.2 us).
+template <int NW>
+__device__ __forceinline__ size_t plane_off(const int* nbs, int bnz, int x, int y, int k) {
+  const int sx = x < 0 ? -1 : (x >= BX ? 1 : 0), sy = y < 0 ? -1 : (y >= BX ? 1 : 0);
+  const size_t cells = (size_t)BX * BX * bnz;
+  return (size_t)nbs[4 + 3 * sy + sx] * NW * cells + ((size_t)k * BX + (y - sy * BX)) * BX + (x - sx * BX);
+}
+
+// Variable 0 of this lane's column cell of plane z, within a block's depth of
+// the block; below / above: its z neighbours, the same for all lanes (z-face
+// kernel: 111 -> 100 us)
+template <int NW>
+__device__ __forceinline__ size_t column_off(int b, int below, int above, int bnz, int t, int z) {
+  const int sb = z < 0 ? below : (z >= bnz ? above : b), zz = z < 0 ? z + bnz : (z >= bnz ? z - bnz : z);
+  return ((size_t)sb * NW * bnz + zz) * (BX * BX) + t;
 }
 
 // z faces of one column per lane, for a chunk of ZC cells: every face whose
@@ -68,6 +84,8 @@ __global__ void __launch_bounds__(NTHREADS, (std::is_same<R, float>::value ? 2 :
   const int tx = threadIdx.x & (BX - 1), ty = threadIdx.x >> 4;
   const size_t cells = (size_t)BX * BX * a.bnz;
   const size_t ntot = (size_t)a.nblocks * cells;
+  const int below = a.nbr[b * 27 + 4], above = a.nbr[b * 27 + 22];
+  auto column = [&](int z) { return column_off<NW>(b, below, above, a.bnz, threadIdx.x, z); };
   R* gz = static_cast<R*>(g.gz);
   // st[s] = cell k-2+s of the face k; ll/lr = lam_out(k-1), (k), in the
   // face precision as the plane kernel's tile holds them; sum[m] = running
@@ -80,10 +98,14 @@ __global__ void __launch_bounds__(NTHREADS, (std::is_same<R, float>::value ? 2 :
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) sum[m][iw] = R(0);
 #pragma unroll
-  for (int s = 0; s < 3; ++s) load_prim<P, R, NDIM>(a, fp, b, tx, ty, k0 - 3 + s, st[s + 1]);
+  for (int s = 0; s < 3; ++s) {
+    double c[NW];
+    load_at<NW>(a.src, column(k0 - 3 + s), cells, c);
+    prim_of<P, R>(c, st[s + 1], fp);
+  }
   auto load_lam_r = [&](int z, R* l) {
     double t[NW];
-    load_lam<NW, NDIM>(a, g.lam_out, b, tx, ty, z, t);
+    load_at<NW>(g.lam_out, column(z), cells, t);
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) l[iw] = R(t[iw]);
   };
@@ -96,8 +118,10 @@ __global__ void __launch_bounds__(NTHREADS, (std::is_same<R, float>::value ? 2 :
       st[2][iw] = st[3][iw];
       ll[iw] = lr[iw];
     }
-    load_prim<P, R, NDIM>(a, fp, b, tx, ty, k + 1, st[3]);
+    double c[NW];
+    load_at<NW>(a.src, column(k + 1), cells, c);
     load_lam_r(k, lr);
+    prim_of<P, R>(c, st[3], fp);
     R mu[NW];
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) mu[iw] = R(a.dq[2] * (double(ll[iw]) - double(lr[iw])));
@@ -162,16 +186,13 @@ __device__ __forceinline__ void glm_source_rev(const SweepArgs& a, const FVParam
     const size_t cells = (size_t)BX * BX * a.bnz;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      int x = tx, y = ty, z = k + 2 * n - 1;
-      double sign;
-      const int sb = locate<NDIM>(a, b, x, y, z, sign);
-      const size_t off = (size_t)sb * P::NW * cells + ((size_t)z * BX + y) * BX + x;
+      const size_t off = column_off<P::NW>(b, a.nbr[b * 27 + 4], a.nbr[b * 27 + 22], a.bnz, ty * BX + tx, k + 2 * n - 1);
 #pragma unroll
       for (int q = 0; q < ND; ++q) {
-        Bn[2][n][q] = double(R(sign * a.src[off + (MAG + q) * cells]));
+        Bn[2][n][q] = double(R(a.src[off + (MAG + q) * cells]));
         lm[2][n][q] = g.lam_out[off + (MOM + q) * cells];
       }
-      psin[2][n] = double(R(sign * a.src[off + S * cells]));
+      psin[2][n] = double(R(a.src[off + S * cells]));
       le[2][n] = g.lam_out[off + E * cells];
     }
   }
@@ -217,9 +238,11 @@ __global__ void __launch_bounds__(NTHREADS, (kAdjWaves<P, R, LIM>))
   // per face round (stencil position s = 0..3): within a pass the faces of
   // a round write distinct cells, so the order of the sums is fixed
   __shared__ double Acc[NW][BX * BX];
+  __shared__ int nbs[9];
   const int b = blockIdx.x / a.bnz, k = blockIdx.x % a.bnz;
   if (b >= a.nblocks) return;
   const int t = threadIdx.x;
+  if (t < 9) nbs[t] = NDIM == 3 ? a.nbr[b * 27 + 9 + t] : a.nbr[b * 9 + t];
   const int tx = t & (BX - 1), ty = t >> 4;
   const size_t cells = (size_t)BX * BX * a.bnz;
   const size_t o = (size_t)b * NW * cells + ((size_t)k * BX + ty) * BX + tx;
@@ -239,22 +262,33 @@ __global__ void __launch_bounds__(NTHREADS, (kAdjWaves<P, R, LIM>))
       zs[iw] = R(0);
     }
   }
-  for (int i = t; i < AW * AW; i += NTHREADS) {
-    const int x = i % AW - AH, y = i / AW - AH;
-    if ((x < 0 || x >= BX) && (y < 0 || y >= BX)) continue;
+  __syncthreads();
+  // Both rounds of each tile are loaded before the first is stored; the lanes
+  // of the unused corners and past the tile repeat the own cell's loads.
+  auto stage_tile = [&](auto Hc, const double* __restrict__ w, auto store) {
+    constexpr int H = decltype(Hc)::value, W = BX + 2 * H, NR = (W * W + NTHREADS - 1) / NTHREADS;
+    double c[NR][NW];
+    bool on[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int i = t + r * NTHREADS, x = i % W - H, y = i / W - H;
+      on[r] = i < W * W && !((x < 0 || x >= BX) && (y < 0 || y >= BX));
+      load_at<NW>(w, plane_off<NW>(nbs, a.bnz, on[r] ? x : tx, on[r] ? y : ty, k), cells, c[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (on[r]) store(t + r * NTHREADS, c[r]);
+  };
+  stage_tile(std::integral_constant<int, AH>(), a.src, [&](int i, const double* c) {
     R w[NW];
-    load_prim<P, R, NDIM>(a, fp, b, x, y, k, w);
+    prim_of<P, R>(c, w, fp);
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) Wl[iw][i] = w[iw];
-  }
-  for (int i = t; i < LW * LW; i += NTHREADS) {
-    const int x = i % LW - LH, y = i / LW - LH;
-    if ((x < 0 || x >= BX) && (y < 0 || y >= BX)) continue;
-    double l[NW];
-    load_lam<NW, NDIM>(a, g.lam_out, b, x, y, k, l);
+  });
+  stage_tile(std::integral_constant<int, LH>(), g.lam_out, [&](int i, const double* c) {
 #pragma unroll
-    for (int iw = 0; iw < NW; ++iw) Ll[iw][i] = R(l[iw]);
-  }
+    for (int iw = 0; iw < NW; ++iw) Ll[iw][i] = R(c[iw]);
+  });
   double acc[NW];
 #pragma unroll
   for (int iw = 0; iw < NW; ++iw) {
