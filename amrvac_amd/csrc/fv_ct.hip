@@ -4,20 +4,20 @@
 // One stage is two launches:
 //   ct_face_kernel    every face flux of the block plus transverse_ghost_cells
 //                     rows (finite_volume src/mod_finite_volume.t:183-190 with
-//                     mhd_modify_wLR :6338-6345), with the face data the edge
-//                     fields need (mhd_get_ct_velocity_* src/mhd/
-//                     mod_mhd_phys.t:3261-3326), into a per-block face buffer;
+//                     mhd_modify_wLR :6338-6345), the flux-divergence update
+//                     of the cells from them, and what the edge fields need
+//                     (mhd_get_ct_velocity_* src/mhd/mod_mhd_phys.t:3261-3326)
+//                     into a per-block face buffer;
 //   ct_update_kernel  edge electric fields (mhd_update_faces_average /
-//                     _contact / _hll :6951-7479), the face-field update, the
-//                     flux-divergence update of the cells, and the cell field
-//                     from the faces (mhd_face_to_center :7586-7648);
+//                     _contact / _hll :6951-7479), the face-field update and
+//                     the cell field from the faces (mhd_face_to_center
+//                     :7586-7648);
 //   the new face field then replaces psb's (the shared face of two blocks
 //                     is computed by both; each stores its upper faces).
 //
 // Face field layout: ws[nb][2][16][16], component d of cell (i, j) is the
-// field on the upper d face of that cell; a face buffer holds per block and
-// direction a 20 x 20 grid (faces -2..17 in both indices) of CT_FK values:
-// the NW unscaled fluxes, then vnorm, cbarmin, cbarmax, vbarC(1), vbarC(2).
+// field on the upper d face of that cell; a face buffer holds 20 x 20 grids
+// (faces or cells -2..17 in both indices) per block.
 #include "fv_ct_common.h"
 
 namespace FV_NS {
@@ -25,56 +25,68 @@ namespace {
 
 using fvc::BX;
 constexpr int CTG = 20;            // face grid edge
-// per block, in doubles: the fluxes [2][NW][20][20] in the face precision
-// (an FP32 flux is stored as the FP32 value it is), then the face data of
-// the edge fields [2][5][20][20] in FP64
+// per block, in doubles: the fluxes of the transverse field component [2][20][20]
+// in the face precision (an FP32 flux is stored as the FP32 value it is), then
+// in FP64 the face data of the edge fields [2][4][20][20] and b x v along z at
+// cell centres [20][20] (uct_contact)
 template <class P>
 struct CtLayout {
-  static constexpr int FK = P::NW + 5;
-  static constexpr int VN = 0, CBMIN = 1, CBMAX = 2, VB1 = 3, VB2 = 4;
+  static constexpr int VN = 0, CBMIN = 0, CBMAX = 1, VB1 = 2, VB2 = 3;
   static constexpr size_t K = (size_t)CTG * CTG;
-  static constexpr size_t per_block = 2 * (size_t)FK * K;
+  static constexpr size_t data = 2 * K, ecc = data + 8 * K, per_block = ecc + K;
 };
 
-__device__ __forceinline__ double ws_at(const SweepArgs& a, const double* ws, int b, int d, int x, int y) {
-  int z = 0;
-  double sign;
-  const int sb = locate<2>(a, b, x, y, z, sign);
-  return ws[((size_t)sb * 2 + d) * BX * BX + (size_t)y * BX + x];
+// A cell or face of a block or beside it, by its owner.  nbs: the block's 9
+// neighbours in LDS (the level is periodic: all exist)
+struct Owner2 {
+  int b, c;
+  __device__ __forceinline__ Owner2(const int* nbs, int x, int y) {
+    const int sx = x < 0 ? -1 : (x >= BX ? 1 : 0), sy = y < 0 ? -1 : (y >= BX ? 1 : 0);
+    b = nbs[4 + 3 * sy + sx];
+    c = (y - sy * BX) * BX + (x - sx * BX);
+  }
+};
+__device__ __forceinline__ void load_neighbours2(const SweepArgs& a, int b, int* nbs) {
+  if (threadIdx.x < 9) nbs[threadIdx.x] = a.nbr[(size_t)b * 9 + threadIdx.x];
+}
+
+__device__ __forceinline__ double ws_at(const double* ws, const Owner2& o, int d) {
+  return ws[((size_t)o.b * 2 + d) * BX * BX + o.c];
 }
 
 // the face field a slot combination gives (the RK initial state of psb)
-__device__ __forceinline__ double ws_comb(const SweepArgs& a, const CtArgs& t, int mode, int b, int d, int x,
-                                          int y) {
-  if (mode == 0) return ws_at(a, t.ws_dst, b, d, x, y);
-  if (mode == 1) return ws_at(a, t.ws_base, b, d, x, y);
-  if (mode == 2) return a.comb_a * ws_at(a, t.ws_base, b, d, x, y) + a.comb_b * ws_at(a, t.ws_src, b, d, x, y);
-  return ws_at(a, t.ws_src, b, d, x, y);
-}
-
-template <class P>
-__device__ __forceinline__ void prim_at(const SweepArgs& a, int b, int x, int y, const FVParams& fp, double* w) {
-  double c[P::NW];
-  load_cons_at<P, 2>(a, b, x, y, 0, c);
-  to_prim<P>(c, w, fp);
+__device__ __forceinline__ double ws_comb(const SweepArgs& a, const CtArgs& t, int mode, const Owner2& o, int d) {
+  if (mode == 0) return ws_at(t.ws_dst, o, d);
+  if (mode == 1) return ws_at(t.ws_base, o, d);
+  if (mode == 2) return a.comb_a * ws_at(t.ws_base, o, d) + a.comb_b * ws_at(t.ws_src, o, d);
+  return ws_at(t.ws_src, o, d);
 }
 
 constexpr int CTS = BX + 4;  // staged cells -2..17 per direction
 
 // the stage input's face field of faces -2..17 of a block, staged in LDS
-__device__ __forceinline__ void stage_ws(const SweepArgs& a, const CtArgs& t, int b, double* wsl) {
+__device__ __forceinline__ void stage_ws(const CtArgs& t, const int* nbs, double* wsl) {
   for (int q = threadIdx.x; q < 2 * CTS * CTS; q += fvc::NTHREADS) {
     const int d = q / (CTS * CTS), r = q % (CTS * CTS);
-    wsl[q] = ws_at(a, t.ws_src, b, d, r % CTS - 2, r / CTS - 2);
+    wsl[q] = ws_at(t.ws_src, Owner2(nbs, r % CTS - 2, r / CTS - 2), d);
   }
 }
 __device__ __forceinline__ double wsl_at(const double* wsl, int d, int x, int y) {
   return wsl[d * CTS * CTS + (y + 2) * CTS + (x + 2)];
 }
 
+constexpr int NE = BX + 1;  // faces and edges -1..15
+
+// the variables updated from their fluxes: all but the two field components
+// that come from the faces; -1 for those
+template <class P>
+__device__ __forceinline__ constexpr int flux_var(int iw) {
+  return iw < P::MAG ? iw : (iw < P::MAG + 2 ? -1 : iw - 2);
+}
+
 template <class P, class R, int RIEM, int LIM, int ID>
 __device__ void ct_one_face(const SweepArgs& a, const CtArgs& t, const FVParams& fp, const R* lds,
-                            const double* wsl, int b, int i, int j, int& crash) {
+                            const double* wsl, const int* nbs, R (*fl)[NE * BX], int b, int i, int j, int& crash) {
   using L = CtLayout<P>;
   constexpr int NW = P::NW;
   R st[4][NW];
@@ -88,19 +100,23 @@ __device__ void ct_one_face(const SweepArgs& a, const CtArgs& t, const FVParams&
   }
   CtIO io;
   io.bn = wsl_at(wsl, ID, i, j);
-  if constexpr (RIEM == RIEM_HLLD)
-    io.bx = t.bx_mode < 0 ? ws_at(a, t.ws_block, b, ID, i, j) : ws_comb(a, t, t.bx_mode, b, ID, i, j);
+  if constexpr (RIEM == RIEM_HLLD) {
+    const Owner2 o(nbs, i, j);
+    io.bx = t.bx_mode < 0 ? ws_at(t.ws_block, o, ID) : ws_comb(a, t, t.bx_mode, o, ID);
+  }
   R fC[NW];
   face_flux<P, R, RIEM, ID, LIM, 2, true>(st, fp, R(0), fC, crash, &io);
   constexpr size_t K = L::K;
   const size_t c = (size_t)(j + 2) * CTG + (i + 2);
-  R* fr = reinterpret_cast<R*>(t.faces + (size_t)b * L::per_block) + (size_t)ID * NW * K + c;
+  // the edge fields take the transverse component's flux
+  reinterpret_cast<R*>(t.faces + (size_t)b * L::per_block)[(size_t)ID * K + c] = fC[P::MAG + 1 - ID];
+  if (ID == 0 ? (j >= 0 && j < BX) : (i >= 0 && i < BX)) {
+    const int q = ID == 0 ? j * NE + i + 1 : (j + 1) * BX + i;
 #pragma unroll
-  // the normal field's flux is read by nothing: the edge fields take the
-  // tangential components and the cell field is the face average
-  for (int iw = 0; iw < NW; ++iw)
-    if (iw != P::MAG + ID) fr[iw * K] = fC[iw];
-  double* f = t.faces + (size_t)b * L::per_block + 2 * NW * K + (size_t)ID * 5 * K + c;
+    for (int iw = 0; iw < NW; ++iw)
+      if (flux_var<P>(iw) >= 0) fl[flux_var<P>(iw)][q] = fC[iw];
+  }
+  double* f = t.faces + (size_t)b * L::per_block + L::data + (size_t)ID * 4 * K + c;
   if (t.ct == CT_CONTACT) f[L::VN * K] = 0.5 * (io.vL[ID] + io.vR[ID]);
   if (t.ct == CT_HLL) {
     const double cbmax = io.cmax > 0.0 ? io.cmax : 0.0;
@@ -117,19 +133,34 @@ __device__ void ct_one_face(const SweepArgs& a, const CtArgs& t, const FVParams&
 // one workgroup per block: the primitive state of cells -2..17 (halo from
 // the neighbours) staged in LDS once (in the face precision R: FP64, or FP32
 // for the mixed form), then both directions' faces: -1..15 along the
-// direction, -tgc..15+tgc across it
+// direction, -tgc..15+tgc across it.  The fluxes of the block's own faces stay
+// in LDS for the update of the cells; to HBM goes only what the edge fields
+// need (with all fluxes and the update in the second kernel that one was bound
+// by their traffic; 1024 x 512, FP64: 45 + 38 -> 54 + 12 us).
 template <class P, class R, int RIEM, int LIM>
 __global__ void __launch_bounds__(fvc::NTHREADS) ct_face_kernel(SweepArgs a, CtArgs t, FVParams fp) {
-  __shared__ R lds[P::NW * CTS * CTS];
+  using L = CtLayout<P>;
+  constexpr int NW = P::NW;
+  __shared__ R lds[NW * CTS * CTS];
+  __shared__ R fl[2][NW - 2][NE * BX];  // x faces [j][i + 1], y faces [j + 1][i]
   __shared__ double wsl[2 * CTS * CTS];
+  __shared__ int nbs[9];
   const int b = wg_block(a.per_xcd);
   if (b >= a.nblocks) return;
-  stage_ws(a, t, b, wsl);
+  load_neighbours2(a, b, nbs);
+  __syncthreads();
+  stage_ws(t, nbs, wsl);
+  const size_t cells = (size_t)BX * BX;
   for (int q = threadIdx.x; q < CTS * CTS; q += fvc::NTHREADS) {
-    double w[P::NW];
-    prim_at<P>(a, b, q % CTS - 2, q / CTS - 2, fp, w);
+    const Owner2 o(nbs, q % CTS - 2, q / CTS - 2);
+    double c[NW], w[NW];
 #pragma unroll
-    for (int iw = 0; iw < P::NW; ++iw) lds[iw * CTS * CTS + q] = R(w[iw]);
+    for (int iw = 0; iw < NW; ++iw) c[iw] = a.src[((size_t)o.b * NW + iw) * cells + o.c];
+    to_prim<P>(c, w, fp);
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw) lds[iw * CTS * CTS + q] = R(w[iw]);
+    if (t.ct == CT_CONTACT)
+      t.faces[(size_t)b * L::per_block + L::ecc + q] = w[P::MAG] * w[P::MOM + 1] - w[P::MAG + 1] * w[P::MOM];
   }
   __syncthreads();
   const int nacross = BX + 2 * t.tgc, nalong = BX + 1, nf = nacross * nalong;
@@ -137,51 +168,78 @@ __global__ void __launch_bounds__(fvc::NTHREADS) ct_face_kernel(SweepArgs a, CtA
   for (int q = threadIdx.x; q < 2 * nf; q += fvc::NTHREADS) {
     const int r = q < nf ? q : q - nf;
     const int along = r % nalong - 1, across = r / nalong - t.tgc;
-    if (q < nf) ct_one_face<P, R, RIEM, LIM, 0>(a, t, fp, lds, wsl, b, along, across, crash);
-    else ct_one_face<P, R, RIEM, LIM, 1>(a, t, fp, lds, wsl, b, across, along, crash);
+    if (q < nf) ct_one_face<P, R, RIEM, LIM, 0>(a, t, fp, lds, wsl, nbs, fl[0], b, along, across, crash);
+    else ct_one_face<P, R, RIEM, LIM, 1>(a, t, fp, lds, wsl, nbs, fl[1], b, across, along, crash);
   }
   if (crash) *a.crash = 1;
+  __syncthreads();
+  // ---- cells: RK initial state + flux divergence
+  const int i = threadIdx.x % BX, j = threadIdx.x / BX;
+  const size_t o = (size_t)b * NW * cells + (size_t)j * BX + i;
+  double acc[NW];
+  if (a.comb_mode == 0 || a.comb_mode == 1) {
+    const double* s0 = a.comb_mode == 0 ? a.dst : a.base;
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw)
+      if (flux_var<P>(iw) >= 0) acc[iw] = s0[o + iw * cells];
+  } else if (a.comb_mode == 2) {
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw)
+      if (flux_var<P>(iw) >= 0) acc[iw] = a.comb_a * a.base[o + iw * cells] + a.comb_b * a.src[o + iw * cells];
+  } else {
+#pragma unroll
+    for (int iw = 0; iw < NW; ++iw)
+      if (flux_var<P>(iw) >= 0) acc[iw] = a.src[o + iw * cells];
+  }
+#pragma unroll
+  for (int iw = 0; iw < NW; ++iw) {
+    const int v = flux_var<P>(iw);
+    if (v < 0) continue;
+    const double fx1 = a.dq[0] * double(fl[0][v][j * NE + i + 1]), fx0 = a.dq[0] * double(fl[0][v][j * NE + i]);
+    acc[iw] = acc[iw] + fx1 - fx0;
+  }
+#pragma unroll
+  for (int iw = 0; iw < NW; ++iw) {
+    const int v = flux_var<P>(iw);
+    if (v < 0) continue;
+    const double fy1 = a.dq[1] * double(fl[1][v][(j + 1) * BX + i]), fy0 = a.dq[1] * double(fl[1][v][j * BX + i]);
+    acc[iw] = acc[iw] + fy1 - fy0;
+  }
+#pragma unroll
+  for (int iw = 0; iw < NW; ++iw)
+    if (flux_var<P>(iw) >= 0) a.dst[o + iw * cells] = acc[iw];
 }
 
-// flux iw through the dim faces (stored in the face precision R)
+// transverse field's flux through the dim faces (stored in the face precision R)
 template <class P, class R>
-__device__ __forceinline__ double fget(const CtArgs& t, int b, int dim, int iw, int i, int j) {
+__device__ __forceinline__ double fget(const CtArgs& t, int b, int dim, int i, int j) {
   using L = CtLayout<P>;
   const R* f = reinterpret_cast<const R*>(t.faces + (size_t)b * L::per_block);
-  return double(f[((size_t)dim * P::NW + iw) * L::K + (size_t)(j + 2) * CTG + (i + 2)]);
+  return double(f[(size_t)dim * L::K + (size_t)(j + 2) * CTG + (i + 2)]);
 }
 
 // face datum k (VN .. VB2) of the dim faces (FP64)
 template <class P>
 __device__ __forceinline__ double dget(const CtArgs& t, int b, int dim, int k, int i, int j) {
   using L = CtLayout<P>;
-  return t.faces[(size_t)b * L::per_block + 2 * P::NW * L::K + ((size_t)dim * 5 + k) * L::K + (size_t)(j + 2) * CTG +
-                 (i + 2)];
+  return t.faces[(size_t)b * L::per_block + L::data + ((size_t)dim * 4 + k) * L::K + (size_t)(j + 2) * CTG + (i + 2)];
 }
 
 template <class P, class R, int LIM>
 __global__ void __launch_bounds__(fvc::NTHREADS) ct_update_kernel(SweepArgs a, CtArgs t, FVParams fp) {
   using L = CtLayout<P>;
   constexpr int NW = P::NW, B1 = P::MAG, B2 = P::MAG + 1;
-  constexpr int NE = BX + 1;  // edges -1..15
   __shared__ double fE[NE * NE];
   __shared__ double wsx[NE * BX];  // x faces i = -1..15, rows 0..15
   __shared__ double wsy[BX * NE];  // y faces rows j = -1..15, columns 0..15
-  __shared__ double ecc[(BX + 2) * (BX + 2)];  // cells -1..16
   __shared__ double wsl[2 * CTS * CTS];         // stage input's faces -2..17 (uct_hll)
+  __shared__ int nbs[9];
   const int b = wg_block(a.per_xcd);
   if (b >= a.nblocks) return;
+  load_neighbours2(a, b, nbs);
+  __syncthreads();
   if (t.ct == CT_HLL) {
-    stage_ws(a, t, b, wsl);
-    __syncthreads();
-  }
-  if (t.ct == CT_CONTACT) {
-    for (int q = threadIdx.x; q < (BX + 2) * (BX + 2); q += fvc::NTHREADS) {
-      const int x = q % (BX + 2) - 1, y = q / (BX + 2) - 1;
-      double w[NW];
-      prim_at<P>(a, b, x, y, fp, w);
-      ecc[q] = w[P::MAG] * w[P::MOM + 1] - w[P::MAG + 1] * w[P::MOM];
-    }
+    stage_ws(t, nbs, wsl);
     __syncthreads();
   }
   // ---- edge electric fields (along z, at the upper x/y corner of cell (i, j))
@@ -190,11 +248,12 @@ __global__ void __launch_bounds__(fvc::NTHREADS) ct_update_kernel(SweepArgs a, C
     double e;
     if (t.ct != CT_HLL) {
       // fC(b1) through y faces, fC(b2) through x faces
-      const double fy0 = fget<P, R>(t, b, 1, B1, i, j), fy1 = fget<P, R>(t, b, 1, B1, i + 1, j);
-      const double fx0 = fget<P, R>(t, b, 0, B2, i, j), fx1 = fget<P, R>(t, b, 0, B2, i, j + 1);
+      const double fy0 = fget<P, R>(t, b, 1, i, j), fy1 = fget<P, R>(t, b, 1, i + 1, j);
+      const double fx0 = fget<P, R>(t, b, 0, i, j), fx1 = fget<P, R>(t, b, 0, i, j + 1);
       e = 0.25 * (fy0 + fy1 - fx0 - fx1);
       if (t.ct == CT_CONTACT) {
-        auto E = [&](int x, int y) { return ecc[(y + 1) * (BX + 2) + (x + 1)]; };
+        const double* ecc = t.faces + (size_t)b * L::per_block + L::ecc;
+        auto E = [&](int x, int y) { return ecc[(y + 2) * CTG + (x + 2)]; };
         const double vx0 = dget<P>(t, b, 0, L::VN, i, j), vx1 = dget<P>(t, b, 0, L::VN, i, j + 1);
         const double vy0 = dget<P>(t, b, 1, L::VN, i, j), vy1 = dget<P>(t, b, 1, L::VN, i + 1, j);
         // first pair: y-face fluxes of b1 at (i, j), (i+1, j)
@@ -259,52 +318,25 @@ __global__ void __launch_bounds__(fvc::NTHREADS) ct_update_kernel(SweepArgs a, C
     {  // x face (i, j), i = -1..15
       const int i = q % NE - 1, j = q / NE;
       const double circ = 0.0 + (FE(i, j) - FE(i, j - 1));
-      const double v = ws_comb(a, t, a.comb_mode, b, 0, i, j) - circ / sCx;
+      const double v = ws_comb(a, t, a.comb_mode, Owner2(nbs, i, j), 0) - circ / sCx;
       wsx[j * NE + (i + 1)] = v;
       if (i >= 0) t.ws_new[((size_t)b * 2 + 0) * BX * BX + (size_t)j * BX + i] = v;
     }
     {  // y face (i, j), j = -1..15
       const int i = q % BX, j = q / BX - 1;
       const double circ = 0.0 - (FE(i, j) - FE(i - 1, j));
-      const double v = ws_comb(a, t, a.comb_mode, b, 1, i, j) - circ / sCy;
+      const double v = ws_comb(a, t, a.comb_mode, Owner2(nbs, i, j), 1) - circ / sCy;
       wsy[(j + 1) * BX + i] = v;
       if (j >= 0) t.ws_new[((size_t)b * 2 + 1) * BX * BX + (size_t)j * BX + i] = v;
     }
   }
   __syncthreads();
-  // ---- cells: RK initial state + flux divergence, then the field from the faces
+  // ---- cells: the field from the faces
   const int i = threadIdx.x % BX, j = threadIdx.x / BX;
   const size_t cells = (size_t)BX * BX;
   const size_t o = (size_t)b * NW * cells + (size_t)j * BX + i;
-  double acc[NW];
-  if (a.comb_mode == 0 || a.comb_mode == 1) {
-    const double* s0 = a.comb_mode == 0 ? a.dst : a.base;
-#pragma unroll
-    for (int iw = 0; iw < NW; ++iw) acc[iw] = s0[o + iw * cells];
-  } else if (a.comb_mode == 2) {
-#pragma unroll
-    for (int iw = 0; iw < NW; ++iw) acc[iw] = a.comb_a * a.base[o + iw * cells] + a.comb_b * a.src[o + iw * cells];
-  } else {
-#pragma unroll
-    for (int iw = 0; iw < NW; ++iw) acc[iw] = a.src[o + iw * cells];
-  }
-  // B1 and B2 come from the faces below, B3 from its fluxes
-#pragma unroll
-  for (int iw = 0; iw < NW; ++iw) {
-    if (iw == B1 || iw == B2) continue;
-    const double fx1 = a.dq[0] * fget<P, R>(t, b, 0, iw, i, j), fx0 = a.dq[0] * fget<P, R>(t, b, 0, iw, i - 1, j);
-    acc[iw] = acc[iw] + fx1 - fx0;
-  }
-#pragma unroll
-  for (int iw = 0; iw < NW; ++iw) {
-    if (iw == B1 || iw == B2) continue;
-    const double fy1 = a.dq[1] * fget<P, R>(t, b, 1, iw, i, j), fy0 = a.dq[1] * fget<P, R>(t, b, 1, iw, i, j - 1);
-    acc[iw] = acc[iw] + fy1 - fy0;
-  }
-  acc[B1] = 0.5 / sCx * (wsx[j * NE + (i + 1)] * sCx + wsx[j * NE + i] * sCx);
-  acc[B2] = 0.5 / sCy * (wsy[(j + 1) * BX + i] * sCy + wsy[j * BX + i] * sCy);
-#pragma unroll
-  for (int iw = 0; iw < NW; ++iw) a.dst[o + iw * cells] = acc[iw];
+  a.dst[o + B1 * cells] = 0.5 / sCx * (wsx[j * NE + (i + 1)] * sCx + wsx[j * NE + i] * sCx);
+  a.dst[o + B2 * cells] = 0.5 / sCy * (wsy[(j + 1) * BX + i] * sCy + wsy[j * BX + i] * sCy);
 }
 
 template <class P, int RIEM, int LIM>
