@@ -650,7 +650,39 @@ sweep_kernel(SweepArgs a, FVParams fp0, CTA ct) {
       // to plane, so that the co-resident workgroups' heavy waves spread
       // over the SIMDs (measured 1.6% faster; the FP32 form is not helped)
       const int t0 = std::is_same<R, double>::value ? (tid + 64 * (k & 3)) % NTHREADS : tid;
-      for (int t = t0; t < NSLOT; t += NTHREADS) {
+      // Where one list of x and y faces takes fewer passes of the workgroup than
+      // two padded ones (8^2 cross-sections: 3 instead of 4), the y faces are
+      // computed as x faces of the stencil with the first two components
+      // swapped: the same operations, sums of two terms in the other order.
+      // (16^2: 9 wave passes instead of 10, measured no faster.)  HLLD's
+      // transverse components are not symmetric in that order.
+      constexpr bool SWAP = NDIM == 3 && std::is_same<R, double>::value && !CT && RIEM != RIEM_HLLD &&
+                            (2 * NXF + NTHREADS - 1) / NTHREADS < (NSLOT + NTHREADS - 1) / NTHREADS;
+      if constexpr (SWAP) {
+        for (int t = tid; t < 2 * NXF; t += NTHREADS) {
+          const int isy = t >= NXF, u = isy ? t - NXF : t;
+          const int r = u / (BX + 1), f = u % (BX + 1);  // row or column, face between f-1 and f
+          auto comp = [&](int iw) {
+            const int v = P::MHD && iw >= P::MAG ? P::MAG : P::MOM;
+            return iw == v ? v + isy : (iw == v + 1 ? v + 1 - isy : iw);
+          };
+          const R* p = &sp[0][0][0] + (isy ? f * PX + r + NG : (r + NG) * PX + f);
+          const int step = isy ? PX : 1;
+          R st[2 * NG][NW];
+#pragma unroll
+          for (int s = 0; s < 2 * NG; ++s)
+#pragma unroll
+            for (int iw = 0; iw < NW; ++iw) st[s][iw] = p[comp(iw) * (PX * PX) + s * step];
+          FVParams fq = fp;
+          fq.rdelinv[0] = isy ? fp.rdelinv[1] : fp.rdelinv[0];
+          fq.cada3k[0] = isy ? fp.cada3k[1] : fp.cada3k[0];
+          R fc[NW];
+          face_flux<P, R, RIEM, 0, LIM, NG>(st, fq, ch, fc, crash);
+          R* o = isy ? &fys[0][f][r] : &fxs[0][r][f];
+#pragma unroll
+          for (int iw = 0; iw < NW; ++iw) o[comp(iw) * (BX * (BX + 1))] = fc[iw];
+        }
+      } else for (int t = t0; t < NSLOT; t += NTHREADS) {
         if (t < NXF) {
           const int y = t / (BX + 1), f = t % (BX + 1);  // face between f-1 and f
           R st[2 * NG][NW];
