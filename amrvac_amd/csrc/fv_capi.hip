@@ -1626,19 +1626,21 @@ static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, doub
 // and the window's prologue (about 2 planes' time); two workgroups on a CU
 // take about 1.6 times as long as one.  The split with the smallest of
 //   rounds of workgroups x time of one
-// is taken, in parts of at least 4 planes (105 blocks of 16^3, MHD: 133 us for
-// a stage in one part, 55 us in four).  The mixed form's blocks stay whole: its
-// carried first z face is rounded apart from the others (the compiler's choice
-// of fused products), so a split would change its results.
-static int stage_zc(const amrvac_fv_ctx* c) {
+// is taken (MHD, 105 blocks of 16^3: 133 us for a stage in one part, 55 us in
+// four; two steps of one block: 1159 us in one part, 289 in four, 155 in
+// sixteen; of 256 blocks: 1409 in one, 805 in two).  The mixed form's blocks stay
+// whole: its carried first z face is rounded apart from the others (the
+// compiler's choice of fused products), so a split would change its results;
+// with constrained transport all its faces are rounded alike.
+static int stage_zc(const amrvac_fv_ctx* c, bool ct = false) {
   if (c->cfg.ndim != 3) return 1;
-  if (c->cfg.precision == AMRVAC_FV_PREC_MIXED) return c->bnz;
+  if (c->cfg.precision == AMRVAC_FV_PREC_MIXED && !ct) return c->bnz;
   const int ncu = 256, per_cu = c->bx == 16 ? 2 : 4;
   int best = c->bnz;
   double tbest = 1e30;
-  for (int nch = 1; nch <= 4; nch *= 2) {
+  for (int nch = 1; nch <= c->bnz; nch *= 2) {
     const int zc = c->bnz / nch;
-    if (zc * nch != c->bnz || (nch > 1 && zc < 4)) continue;
+    if (zc * nch != c->bnz) continue;
     const int n = c->nb * nch, full = n / (ncu * per_cu), rest = n % (ncu * per_cu);
     const double two = 1.0 + 0.6 * (per_cu - 1);
     const double t = (full * two + (rest ? 1.0 + 0.6 * ((rest + ncu - 1) / ncu - 1) : 0.0)) * (zc + 2);
@@ -1795,7 +1797,7 @@ static int ct_stage(amrvac_fv_ctx* c, int method, double dtfactor, double dt, in
   a.comb_b = comb_b;
   const double qdt = dtfactor * dt;
   a.qdt = qdt;
-  a.zc = stage_zc(c);
+  a.zc = stage_zc(c, true);
   a.src_al16 = reinterpret_cast<uintptr_t>(a.src) % 16 == 0;
   for (int d = 0; d < 3; ++d) a.dq[d] = -qdt / c->dx[d];
   c->crash_fresh = false;

@@ -578,7 +578,8 @@ __device__ __forceinline__ void cada3_face64(const FVParams& fp, int id, double 
 // changes nothing under the outer one; max(0, min(A, y)) with y >= 0 is the
 // median; and A, y and the limited value are held twice as large, an exact
 // scaling.  12 VALU instructions per side; with branches a limited side took
-// 26, 7 of them the blend's with no lane enabled.
+// 26, 7 of them the blend's with no lane enabled (256^3 MHD-GLM stage, mixed:
+// 1148 -> 1101 us).
 template <class R>
 __device__ __forceinline__ void cada3_face32(const FVParams& fp, int id, R wm, R w0, R w1, R wp, R& wL, R& wR) {
   const R eps = R(1.4901161193847656e-08);  // sqrt(epsilon(1d0))
@@ -869,7 +870,8 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
       wRp[iw] = st[C0 + 1][iw] - R(0.5) * rdw;
     }
   } else if constexpr (LIM == 0) {
-    // the limiter chosen once per face, not per variable
+    // the limiter chosen once per face, not per variable and side (3-D MHD, cada3,
+    // 3186 blocks of 8^3: 411 -> 290 us)
     switch (fp.limiter) {
       case LIM_MINMOD: tvd_states<P, R, ID, LIM_MINMOD, C0>(st, fp, wLp, wRp); break;
       case LIM_WOODWARD: tvd_states<P, R, ID, LIM_WOODWARD, C0>(st, fp, wLp, wRp); break;
