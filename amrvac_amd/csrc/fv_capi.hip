@@ -1178,9 +1178,10 @@ static bool ensure_pin(amrvac_fv_ctx* c, size_t bytes) {
   return true;
 }
 
-// whether any kernel of this configuration sets the small-value flag
+// whether any kernel of this configuration sets the small-value flag: the
+// checks of fix_small_values, and the pressure of HD's cmaxmean bounds
 static bool may_flag_small(const amrvac_fv_ctx* c) {
-  return c->cfg.fix_small_values || (c->cfg.check_small_values && c->cfg.boundspeed == 2);
+  return c->cfg.fix_small_values || (c->cfg.check_small_values && c->cfg.boundspeed == 2 && c->cfg.physics == 1);
 }
 
 // the small-value flag, read back through the pinned buffer

@@ -154,7 +154,8 @@ class DeviceFV:
         bc = np.ascontiguousarray(mesh.bc_codes, dtype=np.int32)
         # whether any kernel of this configuration sets the small-value flag
         self.may_flag_small = bool(par.fix_small_values
-                                   or (par.check_small_values and par.typeboundspeed == "cmaxmean"))
+                                   or (par.check_small_values and par.typeboundspeed == "cmaxmean"
+                                       and par.physics == "hd"))
         self.amr = hasattr(mesh, "ntype")
         if self.amr:  # an AMR forest (amrvac_amd.amr.AMRForest)
             dx1 = np.ascontiguousarray(mesh.dx[1], dtype=np.float64)
