@@ -190,6 +190,25 @@ struct Phys {
 // conversions
 // ---------------------------------------------------------------------------
 
+// v1^2 + v2^2 (+ v3^2).  Which of the first two products the multiply-add takes
+// in is written out: left to the compiler it is chosen for each place a
+// conversion is inlined at, so that a cell and its copy in a neighbour's halo
+// would get pressures that differ in the last bit.
+template <int N>
+__device__ __forceinline__ double sum_sq(const double* v) {
+  if constexpr (kExact) {
+    double s = v[0] * v[0];
+#pragma unroll
+    for (int d = 1; d < N; ++d) s = s + v[d] * v[d];
+    return s;
+  } else {
+    double s = fma(v[0], v[0], v[1] * v[1]);
+#pragma unroll
+    for (int d = 2; d < N; ++d) s = fma(v[d], v[d], s);
+    return s;
+  }
+}
+
 // hd_to_primitive src/hd/mod_hd_phys.t:703-734,
 // mhd_to_primitive_origin src/mhd/mod_mhd_phys.t:1741-1765 (always FP64:
 // the pressure recovery from total energy cancels at low beta)
@@ -200,15 +219,11 @@ __device__ __forceinline__ void to_prim(const double* c, double* w, const FVPara
   const double inv_rho = 1.0 / w[P::RHO];
 #pragma unroll
   for (int d = 0; d < P::NDIR; ++d) w[P::MOM + d] = w[P::MOM + d] * inv_rho;
-  double vsq = w[P::MOM] * w[P::MOM];
-#pragma unroll
-  for (int d = 1; d < P::NDIR; ++d) vsq = vsq + w[P::MOM + d] * w[P::MOM + d];
+  const double vsq = sum_sq<P::NDIR>(w + P::MOM);
   if constexpr (!P::MHD) {
     w[P::E] = (fp.gamma - 1.0) * (w[P::E] - 0.5 * w[P::RHO] * vsq);
   } else {
-    double bsq = w[P::MAG] * w[P::MAG];
-#pragma unroll
-    for (int d = 1; d < P::NDIR; ++d) bsq = bsq + w[P::MAG + d] * w[P::MAG + d];
+    const double bsq = sum_sq<P::NDIR>(w + P::MAG);
     w[P::E] = fp.gamma_1 * (w[P::E] - 0.5 * (w[P::RHO] * vsq + bsq));
   }
 }
