@@ -1005,6 +1005,16 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
       R aL = cmax * inv, aR = -cmin * inv, aD = cmin * aL;
       if (cmin >= R(0)) { aL = R(1); aR = R(0); aD = R(0); }
       else if (cmax <= R(0)) { aL = R(0); aR = R(1); aD = R(0); }
+      // a side of weight 0 that is infinite (its energy flux is then infinite or
+      // NaN) is not read
+      if (__builtin_expect(!(fabs(fL[P::E] + fR[P::E]) < HUGE_VAL), 0)) {
+#pragma unroll
+        for (int iw = 0; iw < NW; ++iw) {
+          if (iw == BTV) continue;
+          if (cmin >= R(0)) { fR[iw] = fL[iw]; wRC[iw] = wLC[iw]; }
+          else if (cmax <= R(0)) { fL[iw] = fR[iw]; wLC[iw] = wRC[iw]; }
+        }
+      }
 #pragma unroll
       for (int iw = 0; iw < NW; ++iw) {
         if (iw == BTV) fC[iw] = -R(fp.tvdlfeps) * R(0.5) * mx2(cmax, R(fabs(cmin))) * (wRC[iw] - wLC[iw]);
