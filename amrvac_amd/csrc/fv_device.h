@@ -251,8 +251,7 @@ __device__ __forceinline__ bool small_cons(const double* c, const FVParams& fp) 
 
 // hd_to_conserved src/hd/mod_hd_phys.t:677-700,
 // mhd_to_conserved_origin src/mhd/mod_mhd_phys.t:1562-1579
-// FUSE_P: the pressure's product is the fused one whatever code surrounds the
-// conversion (else the compiler takes either)
+// FUSE_P: the pressure's product is the fused one (Fused)
 template <class P, class R, bool FUSE_P = false>
 __device__ __forceinline__ void to_cons(R* w, R inv_gamma_1) {
   R vsq = w[P::MOM] * w[P::MOM];
@@ -276,8 +275,7 @@ __device__ __forceinline__ void to_cons(R* w, R inv_gamma_1) {
 
 // hd_get_flux src/hd/mod_hd_phys.t:1097-1146,
 // mhd_get_flux src/mhd/mod_mhd_phys.t:3810-3889 (GLM :3868-3874)
-// PIN_BN: in b.v the normal field's product is not the fused one whatever code
-// surrounds the flux
+// PIN_BN: in b.v the normal field's product is not the fused one (Fused)
 template <class P, class R, int ID, bool PIN_BN = false>
 __device__ __forceinline__ void phys_flux(const R* wC, const R* w, R ch, R* f) {
   const R vn = w[P::MOM + ID];
@@ -618,8 +616,7 @@ __device__ __forceinline__ void cada3_face32(const FVParams& fp, int id, R wm, R
 // WENO5limiter var=1 src/limiter/mod_weno.t:254-377, one variable, face
 // between cells 0 and 1 of the stencil s[-2..3] (passed as s0..s5 =
 // w(i-2)..w(i+3))
-// PIN: 1 and 2 write out which of two products a multiply-add takes in, where
-// the compiler's choice depends on the code around the face (2: GLM's z faces)
+// PIN: 1 and 2 write out which of two products a multiply-add takes in (Fused)
 template <class R, int PIN = 0>
 __device__ __forceinline__ void weno5(R wmm, R wm, R w0, R wp, R wpp, R wppp, R& wl, R& wr) {
   const R bc1 = R(1.0833333333333333), bc2 = R(0.25);
@@ -869,11 +866,41 @@ struct CtIO {
   double cmax, cmin;
 };
 
+// Which product of a sum the multiply-adds of the mixed form's FP32 faces take
+// in.  The compiler may fuse either, chooses anew for each place a face is
+// inlined at, and changes its mind with the code around it.  The rule is that a
+// face keeps the value it had before its kernel was rearranged: where the choice
+// depends on the surroundings it is written out, and all such places are listed
+// here.  An FP32 value that moves by its last bit moves a run by up to 1e-8.
+//
+// FIRST: the z face below a workgroup's first plane, which the block below
+// forms in its march.  For ideal MHD with TVDLF, and with GLM and WENO5, the two
+// were never rounded alike (mass_flux, einfeldt, weno): there the fluxes at
+// block boundaries in z cancel to FP32 rounding only, and a result depends on
+// the blocks' depth to that extent (64 x 64 x 128, 50 steps: the mass moves by
+// 3e-13 and 1.4e-12, with the others and in FP64 by 4e-15).  All other faces two
+// blocks share are formed alike in both.
+template <class P, class R, int ID, int LIM, bool CT, bool FIRST>
+struct Fused {
+  static constexpr bool F32 = std::is_same<R, float>::value, WENO = LIM == LIM_WENO5;
+  // to_cons: the pressure's product
+  static constexpr bool pressure = F32 && (CT || LIM == LIM_CADA3);
+  // weno5 (all variables but the density): 0 as compiled, 1 and 2 its two forms
+  static constexpr int weno = !F32 || P::NDIM != 3 ? 0 : (P::GLM && ID == 2 && !FIRST ? 2 : 1);
+  // phys_flux: b.v without the normal field's product
+  static constexpr bool normal_field = F32 && CT && P::NDIM == 3 && (LIM == LIM_MINMOD || LIM == LIM_VANLEER);
+  // cbounds with TVDLF: the left side's products of Einfeldt's means
+  static constexpr bool einfeldt = F32 && FIRST && WENO && !P::GLM;
+  // TVDLF: the left side's mass flux
+  static constexpr bool mass_flux = F32 && P::MHD && (FIRST || CT) && !(P::GLM && WENO);
+};
+
 template <class P, class R, int RIEM, int ID, int LIM, int NG, bool CT = false, bool FIRST = false>
 __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& fp, R ch, R* fC,
                                           int& crash, CtIO* ctio = nullptr) {
   constexpr int NW = P::NW;
   constexpr int C0 = NG - 1;  // index of cell i in st
+  using Fu = Fused<P, R, ID, LIM, CT, FIRST>;
   R wLp[NW], wRp[NW];
   if constexpr (LIM == LIM_WENO5) {
     R tl[NW], tr[NW];
@@ -884,9 +911,9 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
       if constexpr (kFast64<R>)
         weno5_face64(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
                      tl[iw], tr[iw]);
-      else if (P::NDIM == 3 && std::is_same<R, float>::value && iw > 0)
-        weno5<R, P::GLM && ID == 2 && !FIRST ? 2 : 1>(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
-                       tl[iw], tr[iw]);
+      else if (iw > 0)
+        weno5<R, Fu::weno>(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw],
+                           st[C0 + 3][iw], tl[iw], tr[iw]);
       else
         weno5(st[C0 - 2][iw], st[C0 - 1][iw], st[C0][iw], st[C0 + 1][iw], st[C0 + 2][iw], st[C0 + 3][iw],
               tl[iw], tr[iw]);
@@ -942,9 +969,8 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
   }
 #pragma unroll
   for (int iw = 0; iw < NW; ++iw) { wLC[iw] = wLp[iw]; wRC[iw] = wRp[iw]; }
-  constexpr bool FUSE_P = (CT || LIM == LIM_CADA3) && std::is_same<R, float>::value;
-  to_cons<P, R, FUSE_P>(wLC, inv_g1);
-  to_cons<P, R, FUSE_P>(wRC, inv_g1);
+  to_cons<P, R, Fu::pressure>(wLC, inv_g1);
+  to_cons<P, R, Fu::pressure>(wRC, inv_g1);
   if constexpr (P::GLM && !GLM_FIRST) {
     constexpr int B = P::MAG + ID, S = P::PSI, E = P::E;
     const R dB = wRp[B] - wLp[B];
@@ -974,19 +1000,17 @@ __device__ __forceinline__ void face_flux(const R (*st)[P::NW], const FVParams& 
     }
   }
   R fL[NW], fR[NW];
-  constexpr bool PIN_BN = CT && P::NDIM == 3 && (LIM == LIM_MINMOD || LIM == LIM_VANLEER) && std::is_same<R, float>::value;
-  phys_flux<P, R, ID, PIN_BN>(wLC, wLp, ch, fL);
-  phys_flux<P, R, ID, PIN_BN>(wRC, wRp, ch, fR);
+  phys_flux<P, R, ID, Fu::normal_field>(wLC, wLp, ch, fL);
+  phys_flux<P, R, ID, Fu::normal_field>(wRC, wRp, ch, fR);
   R cmax, cmin = R(0);
   if constexpr (RIEM == RIEM_TVDLF) {
-    constexpr bool PIN = FIRST && LIM == LIM_WENO5 && !P::GLM && std::is_same<R, float>::value;
-    cbounds<P, R, ID, false, PIN>(wLC, wRC, wLp, wRp, fp, cmax, cmin, crash);
+    cbounds<P, R, ID, false, Fu::einfeldt>(wLC, wRC, wLp, wRp, fp, cmax, cmin, crash);
     if constexpr (CT) { ctio->cmax = cmax; ctio->cmin = cmin; }
     const R fac = R(-0.5) * R(fp.tvdlfeps) * cmax;
 #pragma unroll
     for (int iw = 0; iw < NW; ++iw) {
       fC[iw] = R(0.5) * (fL[iw] + fR[iw]);
-      if constexpr ((FIRST || CT) && P::MHD && !(P::GLM && LIM == LIM_WENO5) && std::is_same<R, float>::value)
+      if constexpr (Fu::mass_flux)
         if (iw == P::RHO) fC[iw] = R(0.5) * fma(wLp[P::MOM + ID], wLp[P::RHO], fR[P::RHO]);
       fC[iw] = fC[iw] + fac * (wRC[iw] - wLC[iw]);
     }
