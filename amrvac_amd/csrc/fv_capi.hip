@@ -1886,6 +1886,12 @@ int amrvac_fv_crash(amrvac_fv_ctx* c, int clear, int* crash_out) {
   return AMRVAC_FV_OK;
 }
 
+int amrvac_fv_may_flag_small(amrvac_fv_ctx* c, int* may_out) {
+  if (!c || !may_out) return fail(AMRVAC_FV_EINVAL, "bad argument");
+  *may_out = may_flag_small(c) ? 1 : 0;
+  return AMRVAC_FV_OK;
+}
+
 int amrvac_fv_getdt(amrvac_fv_ctx* c, int slot, double courantpar, double* dtmin_out, double* cmax_out) {
   if (!c || !check_slot(slot)) return fail(AMRVAC_FV_EINVAL, "bad argument");
   if (!c->slot[0]) return fail(AMRVAC_FV_ESTATE, "no mesh");

@@ -178,6 +178,12 @@ int amrvac_fv_download(amrvac_fv_ctx* ctx, int slot, double* w_host);
    resets it. */
 int amrvac_fv_crash(amrvac_fv_ctx* ctx, int clear, int* crash_out);
 
+/* *may_out = 1 if any kernel of this configuration can raise that flag, else
+   0: a time loop need then not call amrvac_fv_crash, which would wait for the
+   stages, before the next amrvac_fv_getdt does.  No counterpart in the
+   reference. */
+int amrvac_fv_may_flag_small(amrvac_fv_ctx* ctx, int* may_out);
+
 /* Replaces: getdt_courant, maxsum (src/mod_dt.t:160-287) over every block,
    with the min over blocks (the MPI_ALLREDUCE of :81-86 on one rank).
    dtmin_out = min_blocks courantpar / max_cells sum_d cmax_d/dx_d;
