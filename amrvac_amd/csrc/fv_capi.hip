@@ -1237,6 +1237,10 @@ int amrvac_fv_init(const amrvac_fv_config* cfg, amrvac_fv_ctx** out) {
       return fail(AMRVAC_FV_EINVAL, "the mixed form needs block_nx(1) = block_nx(2) = 16");
   }
   if (c.ndim == 3 && c.block_nx[2] < 4) return fail(AMRVAC_FV_EINVAL, "block_nx(3) must be at least 4");
+  // the stage kernels address a block's variables by 32-bit byte offsets
+  const size_t nvar = c.physics == 1 ? c.ndir + 2 : 2 * c.ndir + 2 + (c.divb == 1 ? 1 : 0);
+  if (c.ndim == 3 && nvar * c.block_nx[0] * c.block_nx[1] * c.block_nx[2] * sizeof(double) > UINT32_MAX)
+    return fail(AMRVAC_FV_EINVAL, "block_nx(3) too large: a block's variables must take less than 4 GiB");
   if (c.physics == 2 && c.divb == 4 &&
       (c.block_nx[0] + 2) * (c.block_nx[0] + 2) * (c.ndim == 3 ? c.block_nx[2] + 2 : 1) > fv::kLindeLds)
     return fail(AMRVAC_FV_EINVAL, "Linde cleaning: block_nx(3) too large for the div B tile (at most 22 with "

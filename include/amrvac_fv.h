@@ -56,7 +56,8 @@ typedef struct amrvac_fv_config {
   int check_small_values;               /* 1 */
   int nghost;          /* 2, or 3 for weno5 */
   int block_nx[3];     /* interior cells per block; block_nx(1) = block_nx(2)
-                          = 16, or 8 or 10 in 3-D (FP64) */
+                          = 16, or 8 or 10 in 3-D (FP64); a block's
+                          variables take less than 4 GiB */
   int precision;       /* AMRVAC_FV_PREC_* */
   int type_ct;         /* with divb = 8 (constrained transport on a
                           uniform periodic 2-D or 3-D level, ndir = 3,
