@@ -71,6 +71,7 @@ struct amrvac_fv_ctx {
   int nw = 0;
   int nnb = 0;
   int nb = 0;
+  int ncu = 256;     // compute units of the device
   int bx = 16;       // block_nx(1) = block_nx(2)
   int bnz = 1;
   size_t cells = 0;  // interior cells per block
@@ -1273,6 +1274,10 @@ int amrvac_fv_init(const amrvac_fv_config* cfg, amrvac_fv_ctx** out) {
     return fail(AMRVAC_FV_EHIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
   x->own_stream = true;
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
+    x->ncu = ncu;
   const int rc = scratch_address(&x->scratch);
   if (rc != AMRVAC_FV_OK) {
     (void)hipStreamDestroy(x->stream);
@@ -1633,14 +1638,24 @@ static int getdt_core(amrvac_fv_ctx* c, const double* u, double courantpar, doub
 //   rounds of workgroups x time of one
 // is taken (MHD, 105 blocks of 16^3: 133 us for a stage in one part, 55 us in
 // four; two steps of one block: 1159 us in one part, 289 in four, 155 in
-// sixteen; of 256 blocks: 1409 in one, 805 in two).  The mixed form's blocks stay
-// whole: its carried first z face is rounded apart from the others (the
-// compiler's choice of fused products), so a split would change its results;
-// with constrained transport all its faces are rounded alike.
+// sixteen; of 256 blocks: 1409 in one, 805 in two).  The model's two constants
+// were fitted on that kernel; with WENO5, HD, the Hancock predictor, 8^2 and 10^2
+// cross-sections and depths of 8 to 20 no level of 8 to 2048 blocks is slower
+// than in whole blocks (2 steps of WENO5 MHD, 8 blocks: 1250 -> 196 us, 128: 1328
+// -> 633, 640: 3062 -> 2568; 8^2 with cada3, 8: 482 -> 137, 320: 504 -> 312; from
+// 512 blocks of 8^3 or 10^3 on whole ones are taken).  Halves only: a depth of 12
+// or 20 is split into 2 or 4.
+// A part's first z face is formed in another place than inside a march.  The FP64
+// production kernels may round it apart by a last bit.  The mixed form's blocks
+// stay whole, because some of its configurations round that face as FP32 numbers
+// apart (Fused) and its results would move by up to 1e-8; on levels of up to some
+// 200 blocks it is the slower form for that (MHD-GLM cada3, a step: 1 block 336
+// us against 69 in FP64, 105 blocks 365 against 223, 256 blocks 388 against 397).
+// With constrained transport all its faces are rounded alike, and it is split.
 static int stage_zc(const amrvac_fv_ctx* c, bool ct = false) {
   if (c->cfg.ndim != 3) return 1;
   if (c->cfg.precision == AMRVAC_FV_PREC_MIXED && !ct) return c->bnz;
-  const int ncu = 256, per_cu = c->bx == 16 ? 2 : 4;
+  const int ncu = c->ncu, per_cu = c->bx == 16 ? 2 : 4;
   int best = c->bnz;
   double tbest = 1e30;
   for (int nch = 1; nch <= c->bnz; nch *= 2) {
