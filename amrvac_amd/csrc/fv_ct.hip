@@ -136,7 +136,8 @@ __device__ void ct_one_face(const SweepArgs& a, const CtArgs& t, const FVParams&
 // direction, -tgc..15+tgc across it.  The fluxes of the block's own faces stay
 // in LDS for the update of the cells; to HBM goes only what the edge fields
 // need (with all fluxes and the update in the second kernel that one was bound
-// by their traffic; 1024 x 512, FP64: 45 + 38 -> 54 + 12 us).
+// by their traffic; 1024 x 512, FP64: 45 + 38 -> 54 + 12 us; 56 + 12 with cada3's
+// sides exact).
 template <class P, class R, int RIEM, int LIM>
 __global__ void __launch_bounds__(fvc::NTHREADS) ct_face_kernel(SweepArgs a, CtArgs t, FVParams fp) {
   using L = CtLayout<P>;

@@ -134,8 +134,10 @@ __device__ __forceinline__ double div_by(double a, double b, double binv) {
 template <class R>
 constexpr bool kFast64 = !kExact && std::is_same<R, double>::value;
 
-// sqrt(a) and 1/a of a positive a from one reciprocal square root: both
-// within an ulp or two, in 15 issue slots instead of the 23 of fsqrt and frcp.
+// sqrt(a) and 1/a of a positive a from one reciprocal square root, refined by
+// Goldschmidt's iteration (g -> sqrt(a), h -> 1/(2 sqrt(a))) and a Newton step
+// on 1/a: both within an ulp or two, in 15 issue slots instead of the 23 of fsqrt
+// and frcp.
 __device__ __forceinline__ void sqrt_rcp(double a, double& s, double& inv) {
   const double y = __builtin_amdgcn_rsq(a);
   double g = a * y, h = 0.5 * y;
@@ -147,8 +149,9 @@ __device__ __forceinline__ void sqrt_rcp(double a, double& s, double& inv) {
   const double i = t * t;
   inv = fma(i, fma(-a, i, 1.0), i);
 }
-// sqrt of max(a, 1e-300): the root of a difference that rounding may have
-// made zero or negative; no test for zero (the root is then 1e-150)
+// sqrt of max(a, 1e-300), by the same iteration: the root of a difference that
+// rounding may have made zero or negative; no test for zero (the root is then
+// 1e-150)
 __device__ __forceinline__ double sqrt_floor(double a) {
   a = fmax(a, 1.0e-300);
   const double y = __builtin_amdgcn_rsq(a);

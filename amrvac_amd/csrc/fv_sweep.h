@@ -56,9 +56,9 @@ struct SweepArgs {
   const int* fregoff;       // [nb][2*ndim] register offset of a face, -1: none
   int nface;                // transverse cells of a face (register stride)
   int linde;                // Linde's source follows the stage (linde_kernel)
-  // CFL partials of the output (uniform level): per workgroup the max over
-  // cells of sum_d cmax_d/dx_d and of cmax, as getdt_courant needs them;
-  // nullptr: not wanted
+  // CFL partials of the output (uniform level, mixed form): per block, which is
+  // one workgroup, the max over cells of sum_d cmax_d/dx_d and of cmax, as
+  // getdt_courant needs them; nullptr: not wanted
   double* dt_part;
 };
 

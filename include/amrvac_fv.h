@@ -230,7 +230,8 @@ int amrvac_fv_getdt_state(amrvac_fv_ctx* ctx, const double* u, double courantpar
    library (512 KiB per GPU, held until the process ends) instead of the
    context's buffers; at most 32768 blocks (a larger level is rejected).
    All calls on one GPU share that array: calls that overlap on one GPU
-   race. */
+   race.  (Up to 1024 blocks, where the small-value flag cannot be raised,
+   the maxima go to the context's pinned host buffer instead.) */
 int amrvac_fv_getdt_state_noalloc(amrvac_fv_ctx* ctx, const double* u, double courantpar,
                                   double* dtmin_out, double* cmax_out);
 
