@@ -93,6 +93,7 @@ struct amrvac_fv_ctx {
   // production precision): getdt of ps then only reduces them
   double* d_dtp = nullptr;
   bool dt_valid = false;
+  bool closed = false;  // uniform level: every block has all its face neighbours
   bool slot0_exposed = false;  // ps handed out by amrvac_fv_slot_pointer
   double* d_stage = nullptr;  // ghosted staging for download
   std::vector<double> h_stage;
@@ -1382,6 +1383,11 @@ int amrvac_fv_set_mesh(amrvac_fv_ctx* c, int nblocks, const double* dx, const in
   if (c->nws > 0)
     for (int i = 0; i < nblocks * c->nnb; ++i)
       if (neighbor[i] < 0) return fail(AMRVAC_FV_EINVAL, "constrained transport needs a periodic level");
+  c->closed = true;
+  for (int b = 0; b < nblocks; ++b)
+    for (int d = 0, step = 1; d < nd; ++d, step *= 3)
+      for (int sd = -1; sd <= 1; sd += 2)
+        if (neighbor[b * c->nnb + (c->nnb - 1) / 2 + sd * step] < 0) c->closed = false;
   HIPCHK(hipStreamSynchronize(c->stream));
   free_level(c);
   return alloc_level(c, nblocks, nblocks, dx, neighbor, bc);
@@ -2327,6 +2333,8 @@ int amrvac_fv_adjoint1(amrvac_fv_ctx* c, int method, double dtfactor, double dt,
   if (c->amr) return fail(AMRVAC_FV_EINVAL, "the adjoint stage needs a uniform level");
   for (int sd = 0; sd < 2 * c->cfg.ndim; ++sd)
     if (c->bc[sd] != 5) return fail(AMRVAC_FV_EINVAL, "the adjoint stage needs periodic boundaries");
+  // its kernels take a neighbour's block without a look whether there is one
+  if (!c->closed) return fail(AMRVAC_FV_EINVAL, "the adjoint stage needs all neighbours of every block");
   if (c->cfg.boundspeed != 1) return fail(AMRVAC_FV_EINVAL, "the adjoint stage needs Einfeldt bounds");
   if (c->cfg.limiter != 1 && c->cfg.limiter != 5 && c->cfg.limiter != 9)
     return fail(AMRVAC_FV_EINVAL, "the adjoint needs minmod, vanleer or cada3");
