@@ -13,11 +13,8 @@ from amrvac_amd.mesh import UniformMesh
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ndim", [2, 3])
-@pytest.mark.parametrize("face", range(6))
+@pytest.mark.parametrize("ndim,face", [(2, f) for f in range(4)] + [(3, f) for f in range(6)])
 def test_adjoint_refuses_a_missing_neighbour(ndim, face):
-    if face >= 2 * ndim:
-        pytest.skip("no such face")
     print(f"[adjoint open] {ndim}-D face {face}", flush=True)
     par = Par(physics="hd", ndim=ndim, ndir=ndim, gamma=1.4, time_stepper="threestep", flux_scheme="hll",
               limiter="vanleer")
